@@ -48,47 +48,74 @@ __device__ __forceinline__ void update_c(const BatchDesc& d, const BatchBlock& b
   }
 }
 
-// One (block, tile, split) item; on return every thread has passed the tile
-// routine's last barrier, so the LDS buffers may be reused at once.
-template <bool CPLX, int LA, int WM, int WN, bool LEAN>
-__device__ __forceinline__ void batched_item(
-    const BatchDesc& d, const BatchItem& it,
-    typename TileMma<double, CPLX, LA, KMajor, WM, WN, 2, 16>::Smem& sm) {
-  using T = TileMma<double, CPLX, LA, KMajor, WM, WN, 2, 16, LEAN>;
-  const BatchBlock b = d.blocks[it.block];
-  const int row0 = it.tm * T::BM;  // embedded rows
-  const int col0 = it.tn * T::BN;
-  const int64_t kBegin = static_cast<int64_t>(it.s) * b.kSplit;
-  const int64_t kEnd = min(b.Kp, kBegin + b.kSplit);
-  const TileOperands<double> op{b.A, b.B, b.lda, b.ldb, b.m, b.n, d.conjA, d.conjB};
-  dbl4 acc[T::FM][T::FN];
-  T::run(op, row0, col0, kBegin, kEnd, sm, acc);
-  if (b.splits == 1) {
-    T::for_each(row0, col0, b.m, b.n, acc,
-                [&](int i, int j, double re, double im) { update_c<CPLX>(d, b, i, j, re, im); });
-  } else {
-    double* w = d.work + b.workOffset + static_cast<int64_t>(it.s) * b.n * b.Mp;
-    T::for_each(row0, col0, b.m, b.n, acc, [&](int i, int j, double re, double im) {
-      store_work<double, CPLX>(w, b.Mp, i, j, re, im);
-    });
+// Wave tiles of a configuration (see gemm_f64.hip): R = fragments per 32 embedded rows.
+template <bool CPLX, bool CONJ, int LA, int CFG, bool WIDE = false>
+using BatchMma = TileMma<double, CPLX, CONJ, LA, KMajor, (CPLX ? 1 : 2) * (CFG == TileM ? 1 : 2),
+                         CFG == TileM ? 2 : 4, WIDE>;
+
+// One (block, tile, split) item, its tile covered by repM x repN tiles of T; on
+// return every thread has passed the tile routine's last barrier, so the LDS
+// buffers may be reused at once.
+template <typename T, bool CPLX>
+__device__ __forceinline__ void batched_item(const BatchDesc& d, const BatchItem& it, int repM,
+                                             int repN, typename T::Smem& sm) {
+  const BatchBlock& b = d.blocks[uniform(it.block)];
+  const int m = uniform(b.m), n = uniform(b.n), Mp = uniform(b.Mp), s = uniform(it.s);
+  const int64_t kSplit = uniform(b.kSplit);
+  const int64_t kBegin = s * kSplit;
+  const int64_t kEnd = min(uniform(b.Kp), kBegin + kSplit);
+  const TileOperands<double> op{uniform(b.A), uniform(b.B), uniform(b.lda), uniform(b.ldb), m, n};
+  BatchBlock c;  // what update_c reads
+  c.C = uniform(b.C);
+  c.ldc = uniform(b.ldc);
+  const bool flip = T::flip_result(d.conjA, d.conjB);
+  const bool whole = uniform(b.splits) == 1;
+  double* w = d.work + uniform(b.workOffset) + static_cast<int64_t>(s) * n * Mp;
+#pragma unroll 1
+  for (int t = 0; t < repM * repN; ++t) {
+    const int row = (uniform(it.tm) * repM + t % repM) * T::AR;
+    const int col = (uniform(it.tn) * repN + t / repM) * T::BN;
+    if (row >= m || col >= n) continue;
+    typename T::Acc acc;
+    T::run(op, row, col, kBegin, kEnd, sm, acc);
+    if (whole) {
+      T::for_each(row, col, m, n, flip, acc,
+                  [&](int i, int j, double re, double im) { update_c<CPLX>(d, c, i, j, re, im); });
+    } else {
+      T::for_each(row, col, m, n, flip, acc, [&](int i, int j, double re, double im) {
+        store_work<double, CPLX>(w, Mp, i, j, re, im);
+      });
+    }
   }
 }
 
 // Grouped launch: workgroup = item (gridDim.x = number of items).
-template <bool CPLX, int LA, int WM, int WN>
-__global__ void __launch_bounds__(kThreads, 2) batched_gemm_kernel(BatchDesc d) {
-  __shared__ typename TileMma<double, CPLX, LA, KMajor, WM, WN, 2, 16>::Smem sm;
-  batched_item<CPLX, LA, WM, WN, false>(d, d.items[blockIdx.x], sm);
+template <bool CPLX, bool CONJ, int LA, int CFG>
+__global__ void __launch_bounds__(kThreads, CFG == TileM ? 4 : 2) batched_gemm_kernel(BatchDesc d) {
+  using T = BatchMma<CPLX, CONJ, LA, CFG>;
+  __shared__ typename T::Smem sm;
+  batched_item<T, CPLX>(d, d.items[blockIdx.x], 1, 1, sm);
+}
+
+// The grouped launch for blocks with wide rows (tile_wide): every tile as M tiles.
+template <bool CPLX, bool CONJ, int LA, int CFG>
+__global__ void __launch_bounds__(kThreads, 2) batched_gemm_wide_kernel(BatchDesc d) {
+  using T = BatchMma<CPLX, CONJ, LA, TileM, true>;
+  __shared__ typename T::Smem sm;
+  constexpr int REP = CFG == TileM ? 1 : 2;
+  batched_item<T, CPLX>(d, d.items[blockIdx.x], REP, REP, sm);
 }
 
 // Persistent launch: one workgroup per slot works through its static list of
 // items (gridDim.x = number of slots); no workgroup waits for another.
-template <bool CPLX, int LA, int WM, int WN>
-__global__ void __launch_bounds__(kThreads, 2) batched_gemm_persistent_kernel(BatchDesc d) {
-  __shared__ typename TileMma<double, CPLX, LA, KMajor, WM, WN, 2, 16>::Smem sm;
+template <bool CPLX, bool CONJ, int LA, int CFG>
+__global__ void __launch_bounds__(kThreads, CFG == TileM ? 4 : 2)
+    batched_gemm_persistent_kernel(BatchDesc d) {
+  using T = BatchMma<CPLX, CONJ, LA, CFG>;
+  __shared__ typename T::Smem sm;
   const int end = d.slotStart[blockIdx.x + 1];
   for (int i = d.slotStart[blockIdx.x]; i < end; ++i)
-    batched_item<CPLX, LA, WM, WN, true>(d, d.items[d.slotItems[i]], sm);
+    batched_item<T, CPLX>(d, d.items[uniform(d.slotItems[i])], 1, 1, sm);
 }
 
 // AR x BN: element rows and columns of a tile of the GEMM launch.
@@ -115,29 +142,38 @@ __global__ void __launch_bounds__(kThreads) batched_reduce_kernel(BatchDesc d) {
   }
 }
 
-template <bool CPLX, int LA>
-const void* gemm_kernel_for(int cfg, bool persistent) {
-  if (persistent) {
-    if (cfg == TileM)
-      return reinterpret_cast<const void*>(&batched_gemm_persistent_kernel<CPLX, LA, 32, 32>);
-    return reinterpret_cast<const void*>(&batched_gemm_persistent_kernel<CPLX, LA, 64, 64>);
+template <bool CPLX, bool CONJ, int LA, int CFG>
+const void* gemm_kernel_of(BatchDispatch dispatch) {
+  switch (dispatch) {
+    case BatchPersistent:
+      return reinterpret_cast<const void*>(&batched_gemm_persistent_kernel<CPLX, CONJ, LA, CFG>);
+    case BatchWide:
+      return reinterpret_cast<const void*>(&batched_gemm_wide_kernel<CPLX, CONJ, LA, CFG>);
+    default:
+      return reinterpret_cast<const void*>(&batched_gemm_kernel<CPLX, CONJ, LA, CFG>);
   }
-  if (cfg == TileM) return reinterpret_cast<const void*>(&batched_gemm_kernel<CPLX, LA, 32, 32>);
-  return reinterpret_cast<const void*>(&batched_gemm_kernel<CPLX, LA, 64, 64>);
+}
+
+template <bool CPLX, bool CONJ, int LA>
+const void* gemm_kernel_for(int cfg, BatchDispatch dispatch) {
+  return cfg == TileM ? gemm_kernel_of<CPLX, CONJ, LA, TileM>(dispatch)
+                      : gemm_kernel_of<CPLX, CONJ, LA, TileL>(dispatch);
 }
 
 }  // namespace
 
-BatchKernels batched_kernels(bool complex, int layoutA, int cfg, bool persistent) {
+BatchKernels batched_kernels(bool complex, bool conjA, int layoutA, int cfg,
+                             BatchDispatch dispatch) {
   BatchKernels k;
   if (complex) {
-    k.gemm = layoutA == MNMajor ? gemm_kernel_for<true, MNMajor>(cfg, persistent)
-                                : gemm_kernel_for<true, KMajor>(cfg, persistent);
+    k.gemm = layoutA == MNMajor ? gemm_kernel_for<true, false, MNMajor>(cfg, dispatch)
+             : conjA            ? gemm_kernel_for<true, true, KMajor>(cfg, dispatch)
+                                : gemm_kernel_for<true, false, KMajor>(cfg, dispatch);
     k.reduce = cfg == TileM ? reinterpret_cast<const void*>(&batched_reduce_kernel<true, 32, 64>)
                             : reinterpret_cast<const void*>(&batched_reduce_kernel<true, 64, 128>);
   } else {
-    k.gemm = layoutA == MNMajor ? gemm_kernel_for<false, MNMajor>(cfg, persistent)
-                                : gemm_kernel_for<false, KMajor>(cfg, persistent);
+    k.gemm = layoutA == MNMajor ? gemm_kernel_for<false, false, MNMajor>(cfg, dispatch)
+                                : gemm_kernel_for<false, false, KMajor>(cfg, dispatch);
     k.reduce = cfg == TileM ? reinterpret_cast<const void*>(&batched_reduce_kernel<false, 64, 64>)
                             : reinterpret_cast<const void*>(&batched_reduce_kernel<false, 128, 128>);
   }

@@ -3,13 +3,10 @@
 // The kernels compute C <- alpha * opA(A) * opB(B) + beta * C for column-major
 // real or interleaved complex operands of one scalar type (double or float;
 // the FP32 kernels accumulate in FP32, as a single-precision BLAS does). A
-// complex product is run as a real product of the "real embedding": every
-// 16-row MFMA fragment holds the real and the imaginary rows of 8 complex rows
-// of C (FP64: rows 0-7 real, 8-15 imaginary; FP32: rows 2c real, 2c + 1
-// imaginary, following each instruction's accumulator layout), and the reduction index q = 2*l + c runs over the real (c = 0) and
-// imaginary (c = 1) parts of A(l, i) / B(l, j). The complex product is then
-// one real GEMM of size (2m) x n x (2k), i.e. exactly 8*m*n*k flops, with no
-// operand expanded in memory. Split-K partial sums are stored as interleaved
+// complex product is four real products per pair of elements, exactly 8*m*n*k
+// flops, with no operand expanded in memory. Its sizes are given as those of
+// one real GEMM of size (2m) x n x (2k), the "embedded" sizes Mp and Kp:
+// q = 2*l + c runs over the real (c = 0) and imaginary (c = 1) parts. Split-K partial sums are stored as interleaved
 // (re, im) pairs, i.e. in C's own column-major complex layout.
 #pragma once
 
@@ -74,6 +71,15 @@ inline TileShape tile_shape(int cfg) {
     default:
       return {128, 128, 16};
   }
+}
+
+// The tile kernels address a wave's share of a tile with 32-bit lane offsets: 32
+// rows of a K-major operand or 32 reduction indices of an MN-major one. Operands
+// whose leading dimension spreads these over 4 GiB (complex doubles: from 8.1e6
+// elements) take kernels with 64-bit lane addresses, which spend vector
+// instructions on them in every k-block.
+inline bool tile_wide(int64_t ld, int elemBytes) {
+  return 33 * ld * elemBytes >= (int64_t(1) << 32);
 }
 
 }  // namespace spla_amd

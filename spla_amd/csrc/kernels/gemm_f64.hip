@@ -7,20 +7,8 @@
 // operations the engine issues: opA in {N, T, C}, opB in {N, T, C}.
 //
 // Structure of one workgroup (256 threads = 4 wave64):
-//   * a BM x BN tile of the embedded output (see gemm_desc.hpp), split over a
-//     WAVES_M x WAVES_N grid of waves, each owning WM x WN = (WM/16)x(WN/16)
-//     MFMA accumulators of 16x16 scalars;
-//   * the reduction runs over k-blocks of BK embedded elements, double
-//     buffered in LDS with one barrier per k-block; the next block's global
-//     loads are issued before the MFMAs of the current one;
-//   * inside a k-block the reduction index is permuted so that every lane
-//     reads its A and B operands as 16-byte pairs (q = 8*b + 2*kk + step):
-//     A and B use the same permutation, so the sum is unchanged;
-//   * complex: inside each 16-row MFMA fragment, rows 0-7 carry the real and
-//     rows 8-15 the imaginary parts of 8 complex rows of C. The A operand of
-//     an imaginary row reads the partner component of the pair (swap) with a
-//     lane-constant sign, so A and B are staged exactly once and no operand
-//     is expanded in memory; every lane ends up holding whole complex results;
+//   * a tile of the output (sizes in embedded rows, see gemm_desc.hpp), split
+//     over a 2 x 2 grid of waves; the k loop is that of tile_mma.hpp;
 //   * split-K: a split writes its raw partial sums to a workspace; the
 //     reduction kernel adds the splits in a fixed order (bitwise
 //     reproducible) and applies alpha / beta. With one split the epilogue is
@@ -92,48 +80,79 @@ __device__ __forceinline__ void map_block(const GemmDesc& d, int& s, int& tm, in
   tn = inGroup / gsize;
 }
 
-// Body of one workgroup (shared by the FP64 and FP32 kernels).
-template <typename S, bool CPLX, int LA, int LB, int WM, int WN, int WAVES_M, int BK>
-__device__ __forceinline__ void gemm_tile(const GemmDesc& d,
-                                          typename TileMma<S, CPLX, LA, LB, WM, WN, WAVES_M,
-                                                           BK>::Smem& sm) {
-  using T = TileMma<S, CPLX, LA, LB, WM, WN, WAVES_M, BK>;
+// Body of one workgroup (shared by the FP64 and FP32 kernels): one tile of T, or
+// (MULTI) repM x repN of them one after the other.
+template <typename T, typename S, bool CPLX, bool MULTI>
+__device__ __forceinline__ void gemm_tile(const GemmDesc& d, int repM, int repN,
+                                          typename T::Smem& sm) {
   int s, tm, tn;
   map_block(d, s, tm, tn);
-  const int row0 = tm * T::BM;  // embedded rows
-  const int col0 = tn * T::BN;
-  const int arow0 = CPLX ? row0 / 2 : row0;
+  if (!MULTI) repM = repN = 1;
+  const int first = tm * T::AR * repM;
+  const int col0 = tn * T::BN * repN;
   if (d.fillMode != FillFull) {
-    const int64_t nr = min(T::AR, d.m - arow0);
-    const int64_t nc = min(T::BN, d.n - col0);
-    if (!tile_active(d, arow0, col0, nr, nc)) return;
+    const int64_t nr = min(T::AR * repM, d.m - first);
+    const int64_t nc = min(T::BN * repN, d.n - col0);
+    if (!tile_active(d, first, col0, nr, nc)) return;
   }
   const int64_t kBegin = static_cast<int64_t>(s) * d.kSplit;
   const int64_t kEnd = min(d.Kp, kBegin + d.kSplit);
-  const TileOperands<S> op{static_cast<const S*>(d.A), static_cast<const S*>(d.B), d.lda, d.ldb,
-                           d.m, d.n, d.conjA, d.conjB};
-  typename T::Acc acc[T::FM][T::FN];
-  T::run(op, row0, col0, kBegin, kEnd, sm, acc);
-  if (d.splits > 1) {
-    S* w = static_cast<S*>(d.work) + static_cast<int64_t>(s) * d.n * d.Mp;
-    T::for_each(row0, col0, d.m, d.n, acc,
-                [&](int i, int j, S re, S im) { store_work<S, CPLX>(w, d.Mp, i, j, re, im); });
+  const TileOperands<S> op{uniform(static_cast<const S*>(d.A)), uniform(static_cast<const S*>(d.B)),
+                           uniform(d.lda), uniform(d.ldb), uniform(d.m), uniform(d.n)};
+  const bool flip = T::flip_result(d.conjA, d.conjB);
+  S* w = static_cast<S*>(d.work) + static_cast<int64_t>(s) * d.n * d.Mp;
+  auto one = [&](int row, int col) {
+    row = uniform(row);
+    col = uniform(col);
+    typename T::Acc acc;
+    T::run(op, row, col, kBegin, kEnd, sm, acc);
+    if (d.splits > 1) {
+      T::for_each(row, col, d.m, d.n, flip, acc,
+                  [&](int i, int j, S re, S im) { store_work<S, CPLX>(w, d.Mp, i, j, re, im); });
+    } else {
+      T::for_each(row, col, d.m, d.n, flip, acc,
+                  [&](int i, int j, S re, S im) { store_result<S, CPLX>(d, i, j, re, im); });
+    }
+  };
+  if constexpr (!MULTI) {
+    one(first, col0);
   } else {
-    T::for_each(row0, col0, d.m, d.n, acc,
-                [&](int i, int j, S re, S im) { store_result<S, CPLX>(d, i, j, re, im); });
+#pragma unroll 1
+    for (int t = 0; t < repM * repN; ++t) {
+      const int row = first + (t % repM) * T::AR, col = col0 + (t / repM) * T::BN;
+      if (row < d.m && col < d.n) one(row, col);
+    }
   }
 }
 
-template <bool CPLX, int LA, int LB, int WM, int WN, int WAVES_M, int BK, int MINBLOCKS>
+template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN, int MINBLOCKS>
 __global__ void __launch_bounds__(kThreads, MINBLOCKS) gemm_f64_kernel(GemmDesc d) {
-  __shared__ typename TileMma<double, CPLX, LA, LB, WM, WN, WAVES_M, BK>::Smem sm;
-  gemm_tile<double, CPLX, LA, LB, WM, WN, WAVES_M, BK>(d, sm);
+  using T = TileMma<double, CPLX, CONJ, LA, LB, FM, FN>;
+  __shared__ typename T::Smem sm;
+  gemm_tile<T, double, CPLX, false>(d, 1, 1, sm);
 }
 
-template <bool CPLX, int LA, int LB, int WM, int WN, int WAVES_M, int BK, int MINBLOCKS>
+// Tiles of repM x repN of the kernel's own (see launch_layout).
+template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN, bool WIDE>
+__global__ void __launch_bounds__(kThreads, 2) gemm_f64_multi_kernel(GemmDesc d, int repM, int repN) {
+  using T = TileMma<double, CPLX, CONJ, LA, LB, FM, FN, WIDE>;
+  __shared__ typename T::Smem sm;
+  gemm_tile<T, double, CPLX, true>(d, repM, repN, sm);
+}
+
+template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN, int MINBLOCKS>
 __global__ void __launch_bounds__(kThreads, MINBLOCKS) gemm_f32_kernel(GemmDesc d) {
-  __shared__ typename TileMma<float, CPLX, LA, LB, WM, WN, WAVES_M, BK>::Smem sm;
-  gemm_tile<float, CPLX, LA, LB, WM, WN, WAVES_M, BK>(d, sm);
+  using T = TileMma<float, CPLX, CONJ, LA, LB, FM, FN>;
+  __shared__ typename T::Smem sm;
+  gemm_tile<T, float, CPLX, false>(d, 1, 1, sm);
+}
+
+// Tiles of repM x repN of the kernel's own (see launch_layout).
+template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN, bool WIDE>
+__global__ void __launch_bounds__(kThreads, 2) gemm_f32_multi_kernel(GemmDesc d, int repM, int repN) {
+  using T = TileMma<float, CPLX, CONJ, LA, LB, FM, FN, WIDE>;
+  __shared__ typename T::Smem sm;
+  gemm_tile<T, float, CPLX, true>(d, repM, repN, sm);
 }
 
 // Adds the split-K partial sums in split order and applies alpha / beta.
@@ -239,52 +258,81 @@ __global__ void __launch_bounds__(256) scale_kernel(GemmDesc d) {
   }
 }
 
-template <bool F32, bool CPLX, int LA, int LB>
+// Wave tiles: L 64 x 64 embedded rows and columns (two workgroups per CU), M
+// 32 x 32 (four); XL is two L tiles one after the other (128 x 64 wave tiles, one
+// wave per SIMD, keep the compiler moving accumulators between register files).
+// Operands with wide rows (tile_wide) run every shape as M tiles.
+template <bool F32, bool CPLX, bool CONJ, int LA, int LB>
 hipError_t launch_layout(const GemmDesc& d, int cfg, hipStream_t stream) {
+  constexpr int R = CPLX ? 1 : 2;  // fragments per 32 embedded rows
   const dim3 block(kThreads);
   const dim3 grid(static_cast<unsigned>(d.tilesM * d.tilesN * d.splits));
-  if (F32) {
+  const int elem = (F32 ? 4 : 8) * (CPLX ? 2 : 1);
+  if (tile_wide(d.lda, elem) || tile_wide(d.ldb, elem)) {
+    const TileShape ts = tile_shape(cfg), tm = tile_shape(TileM);
+    if constexpr (F32)
+      hipLaunchKernelGGL((gemm_f32_multi_kernel<CPLX, CONJ, LA, LB, R, 2, true>), grid, block, 0,
+                         stream, d, ts.bm / tm.bm, ts.bn / tm.bn);
+    else
+      hipLaunchKernelGGL((gemm_f64_multi_kernel<CPLX, CONJ, LA, LB, R, 2, true>), grid, block, 0,
+                         stream, d, ts.bm / tm.bm, ts.bn / tm.bn);
+    return hipGetLastError();
+  }
+  if constexpr (F32) {
     switch (cfg) {
       case TileM:
-        hipLaunchKernelGGL((gemm_f32_kernel<CPLX, LA, LB, 32, 32, 2, 16, 2>), grid, block, 0,
-                           stream, d);
+        hipLaunchKernelGGL((gemm_f32_kernel<CPLX, CONJ, LA, LB, R, 2, 4>), grid, block, 0, stream,
+                           d);
         break;
       case TileXL:
-        hipLaunchKernelGGL((gemm_f32_kernel<CPLX, LA, LB, 128, 64, 2, 16, 1>), grid, block, 0,
-                           stream, d);
+        hipLaunchKernelGGL((gemm_f32_multi_kernel<CPLX, CONJ, LA, LB, 2 * R, 4, false>), grid,
+                           block, 0, stream, d, 2, 1);
         break;
       default:
-        hipLaunchKernelGGL((gemm_f32_kernel<CPLX, LA, LB, 64, 64, 2, 16, 2>), grid, block, 0,
+        hipLaunchKernelGGL((gemm_f32_kernel<CPLX, CONJ, LA, LB, 2 * R, 4, 2>), grid, block, 0,
                            stream, d);
         break;
     }
-    return hipGetLastError();
-  }
-  switch (cfg) {
-    case TileM:
-      hipLaunchKernelGGL((gemm_f64_kernel<CPLX, LA, LB, 32, 32, 2, 16, 2>), grid, block, 0, stream,
-                         d);
-      break;
-    case TileXL:
-      hipLaunchKernelGGL((gemm_f64_kernel<CPLX, LA, LB, 128, 64, 2, 16, 1>), grid, block, 0,
-                         stream, d);
-      break;
-    default:
-      hipLaunchKernelGGL((gemm_f64_kernel<CPLX, LA, LB, 64, 64, 2, 16, 2>), grid, block, 0, stream,
-                         d);
-      break;
+  } else {
+    switch (cfg) {
+      case TileM:
+        hipLaunchKernelGGL((gemm_f64_kernel<CPLX, CONJ, LA, LB, R, 2, 4>), grid, block, 0, stream,
+                           d);
+        break;
+      case TileXL:
+        hipLaunchKernelGGL((gemm_f64_multi_kernel<CPLX, CONJ, LA, LB, 2 * R, 4, false>), grid,
+                           block, 0, stream, d, 2, 1);
+        break;
+      default:
+        hipLaunchKernelGGL((gemm_f64_kernel<CPLX, CONJ, LA, LB, 2 * R, 4, 2>), grid, block, 0,
+                           stream, d);
+        break;
+    }
   }
   return hipGetLastError();
 }
 
+// A is conjugated only as A^H (K-major), B only as B^H (MN-major): MN-major A
+// times K-major B is never conjugated.
+template <bool F32, bool CPLX, int LA, int LB>
+hipError_t launch_conj(const GemmDesc& d, int cfg, hipStream_t stream) {
+  if constexpr (CPLX && !(LA == MNMajor && LB == KMajor)) {
+    if ((d.conjA != 0) != (d.conjB != 0))
+      return launch_layout<F32, CPLX, true, LA, LB>(d, cfg, stream);
+  } else {
+    if (d.conjA || d.conjB) return hipErrorInvalidValue;
+  }
+  return launch_layout<F32, CPLX, false, LA, LB>(d, cfg, stream);
+}
+
 template <bool F32, bool CPLX>
 hipError_t launch_typed(const GemmDesc& d, int la, int lb, int cfg, hipStream_t stream) {
-  if (la == KMajor && lb == KMajor) return launch_layout<F32, CPLX, KMajor, KMajor>(d, cfg, stream);
+  if (la == KMajor && lb == KMajor) return launch_conj<F32, CPLX, KMajor, KMajor>(d, cfg, stream);
   if (la == KMajor && lb == MNMajor)
-    return launch_layout<F32, CPLX, KMajor, MNMajor>(d, cfg, stream);
+    return launch_conj<F32, CPLX, KMajor, MNMajor>(d, cfg, stream);
   if (la == MNMajor && lb == KMajor)
-    return launch_layout<F32, CPLX, MNMajor, KMajor>(d, cfg, stream);
-  return launch_layout<F32, CPLX, MNMajor, MNMajor>(d, cfg, stream);
+    return launch_conj<F32, CPLX, MNMajor, KMajor>(d, cfg, stream);
+  return launch_conj<F32, CPLX, MNMajor, MNMajor>(d, cfg, stream);
 }
 
 }  // namespace

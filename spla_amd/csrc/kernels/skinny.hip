@@ -162,11 +162,11 @@ __global__ void __launch_bounds__(kWaves * 64, 2) skinny_gemm_kernel(GemmDesc d)
 #pragma unroll
       for (int f = 0; f < FM; ++f)
 #pragma unroll
-        for (int g = 0; g < FN; ++g) acc[f][g] = mfma16x16x4(a0[f], b0[g], acc[f][g]);
+        for (int g = 0; g < FN; ++g) acc[f][g] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[f], b0[g], acc[f][g], 0, 0, 0);
 #pragma unroll
       for (int f = 0; f < FM; ++f)
 #pragma unroll
-        for (int g = 0; g < FN; ++g) acc[f][g] = mfma16x16x4(a1[f], b1[g], acc[f][g]);
+        for (int g = 0; g < FN; ++g) acc[f][g] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[f], b1[g], acc[f][g], 0, 0, 0);
     }
   };
 

@@ -1,14 +1,54 @@
 // MFMA tile routine shared by the single-product kernels (gemm_f64.hip: FP64
-// and FP32, real and complex) and the persistent batched kernel (batched.hip).
+// and FP32, real and complex) and the batched kernels (batched.hip).
 // Device code only; include from HIP translation units.
 //
-// The scalar type S is double (v_mfma_f64_16x16x4_f64) or float
-// (v_mfma_f32_16x16x4_f32). Both instructions take lane l's operands as
-// A[l % 16][l / 16] and B[l / 16][l % 16]; their accumulators differ: lane l
-// holds rows (l / 16) + 4 r (FP64) or 4 (l / 16) + r (FP32), r = 0..3, of
-// column l % 16. A complex product puts the real and imaginary rows of a
-// complex row of C into the same lane: FP64 fragment rows r and r + 8, FP32
-// fragment rows 2 c and 2 c + 1.
+// What bounds it: the matrix cores, and the vector ALU next to them. On gfx950
+// a VALU instruction does not run beside an FP64 or FP32 MFMA of its SIMD: in
+// register-only loops (two waves per SIMD) one v_xor_b32 per MFMA takes
+// v_mfma_f64_16x16x4_f64 from 75.5 to 70.1 TFLOP/s, two to 67.3, four to 64.0
+// (v_mfma_f32_16x16x4_f32: 149, 128, 122, 112), while scalar instructions and
+// one ds_read_b128 per MFMA cost nothing. The k loop is therefore written
+// without vector arithmetic:
+//   * complex operands are not expanded. A fragment holds 16 complex rows (or
+//     columns); a lane's 16-byte chunk gives the real and the imaginary operand
+//     as they lie in memory, and four MFMAs (re re, im im, im re, re im) make
+//     the real and the imaginary accumulators of the same lane. Signs: the FP64
+//     MFMA negates its operand itself; FP32 flips the imaginary part of A, one
+//     VALU instruction for 2 FN MFMAs. A conjugated result is the product of
+//     the other operand's conjugate, so one template bit covers all four
+//     conj(A), conj(B) forms (flip_result negates the imaginary part once, in
+//     the epilogue).
+//   * global addresses are a wave-uniform 64-bit base (scalar unit) plus a
+//     32-bit lane offset that stays the same for the whole reduction.
+//   * rows past the operand's edge are clamped to its last row when the
+//     offsets are made: they only feed outputs that are not stored, so ragged
+//     tiles run the same loop (with per-element checks in the loop the edge
+//     tiles of a 1000 x 1000 x 1e5 product held it at 39 TFLOP/s).
+//   * LDS addresses are one base per operand plus immediate offsets (the two
+//     buffers are unrolled).
+//   * the last, partial k-block takes a separate checked load.
+//
+// Measured against the same tiles with the embedding's swaps and signs, 64-bit
+// addresses and row checks in the loop (one card): complex doubles 2048 x 2048 x
+// 2e5 A^H B 102.3 -> 92.2 ms (72.8 TFLOP/s), 100000 x 4096 x 4096 A B 201.8 ->
+// 176.4 ms (76.1 of the 77.1 a register-only loop reaches), complex floats 2048 x
+// 2048 x 2e5 58.9 -> 45.3 ms (148 of 155), real doubles 1000 x 1000 x 1e5 A^T B
+// (ragged) 5.53 -> 3.59 ms.
+//
+// Layouts. A k-block is 128 bytes of a K-major row (8 complex or 16 real
+// doubles, 16 complex or 32 real floats) in two sub-blocks of four 16-byte
+// chunks; lane group kk = lane / 16 reads chunk kk of its row. MN-major
+// operands lie in LDS as they lie in memory, [reduction index][row]: a 16-byte
+// read there holds VR neighbouring rows of one reduction index, which become
+// the same lane's operands of VR fragments (fragment p covers rows
+// VR * (lane % 16) + p), so nothing is transposed. Both layouts take the
+// reduction index in the same order inside a sub-block (element s of chunk kk).
+//
+// The MFMAs take B as their first operand: D rows are columns of C and a
+// lane's D column is a row of C, so 16 lanes store 16 neighbouring rows of a
+// column of C (128 bytes of doubles, 256 of complex doubles).
+// Accumulators of lane (kk, l16), column l16 of D: D rows kk + 4 r (FP64) or
+// 4 kk + r (FP32), r = 0..3.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -25,610 +65,529 @@ typedef double dbl2 __attribute__((ext_vector_type(2)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
 typedef float flt2 __attribute__((ext_vector_type(2)));
 
+template <typename S, int N>
+struct VecOf {
+  typedef S type __attribute__((ext_vector_type(N)));
+  // as it lies in a caller's matrix: aligned like one scalar
+  typedef S loose __attribute__((ext_vector_type(N), aligned(sizeof(S))));
+};
 template <typename S>
-struct Vec;
-template <>
-struct Vec<double> {
-  using V2 = dbl2;
-  using V4 = dbl4;
+struct VecOf<S, 1> {
+  typedef S type;
+  typedef S loose;
 };
-template <>
-struct Vec<float> {
-  using V2 = flt2;
-  using V4 = flt4;
+
+// Load of one register piece (4, 8 or 16 bytes) at a 32-bit lane offset.
+template <typename P>
+__device__ __forceinline__ P buffer_load(__amdgpu_buffer_rsrc_t rsrc, uint32_t off,
+                                         uint32_t scalarOff) {
+  static_assert(sizeof(P) == 4 || sizeof(P) == 8 || sizeof(P) == 16, "piece of 4, 8 or 16 bytes");
+  if constexpr (sizeof(P) == 16)
+    return __builtin_bit_cast(P, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, scalarOff, 0));
+  else if constexpr (sizeof(P) == 8)
+    return __builtin_bit_cast(P, __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, scalarOff, 0));
+  else
+    return __builtin_bit_cast(P, __builtin_amdgcn_raw_buffer_load_b32(rsrc, off, scalarOff, 0));
+}
+
+template <int N>
+struct Index {
+  static constexpr int value = N;
 };
+
+// The same value in a scalar register: loads through pointers that the kernel's
+// own stores might alias leave wave-uniform values in vector registers.
+template <typename V>
+__device__ __forceinline__ V uniform(V v) {
+  static_assert(sizeof(V) == 4 || sizeof(V) == 8, "one or two registers");
+  if constexpr (sizeof(V) == 4) {
+    return __builtin_bit_cast(
+        V, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(uint32_t, v)));
+  } else {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint64_t lo =
+        static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b)));
+    const uint64_t hi =
+        static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b >> 32)));
+    return __builtin_bit_cast(V, hi << 32 | lo);
+  }
+}
 
 constexpr int kThreads = 256;
-// LDS row padding (elements; even, so that element pairs stay 16-byte aligned).
-// Rows of BK = 16 doubles are 128 bytes. Measured on gfx950 with the
-// bank-conflict counter on the fragment reads (ds_read_b128: 16 rows x 4
-// 16-byte chunks per wave): 160-byte rows read conflict-free, 144-, 176- and
-// 208-byte rows cost 4 conflict cycles per read. 160-byte rows cost 8 cycles on
-// an MN-major store (eight rows, one chunk), which is rarer than the reads of
-// the same tile; they fill the 160 KB of a CU exactly with two real 128 x 128
-// or four real 64 x 64 workgroups. FP32 rows keep 2 floats of padding.
-template <typename S, bool CPLX>
-constexpr int kPadOf = sizeof(S) == 8 ? 4 : 2;
+constexpr int kChunk = 16;      // bytes of one lane's fragment read
+constexpr int kBlockBytes = 128;  // bytes of a K-major row in one k-block
+// Row stride of K-major tiles in LDS, measured with the bank-conflict counter on
+// the fragment reads (ds_read_b128: 16 rows x 4 chunks per wave): 160-byte rows
+// read conflict-free, 144-, 176- and 208-byte rows cost 4 conflict cycles.
+constexpr int kRowBytes = 160;
 
-__device__ __forceinline__ double flip_sign(double x, uint32_t hiMask) {
-  uint64_t b = __builtin_bit_cast(uint64_t, x);
-  b ^= static_cast<uint64_t>(hiMask) << 32;
-  return __builtin_bit_cast(double, b);
+// D = B-operand x A-operand + D; NEG negates the A operand.
+template <bool NEG>
+__device__ __forceinline__ dbl4 mfma16x16x4(double b, double a, dbl4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, c, 0, 0, NEG ? 2 : 0);
 }
-__device__ __forceinline__ float flip_sign(float x, uint32_t mask) {
-  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) ^ mask);
+template <bool NEG>
+__device__ __forceinline__ flt4 mfma16x16x4(float b, float a, flt4 c) {
+  static_assert(!NEG, "the FP32 MFMA has no operand negation");
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(b, a, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ dbl4 mfma16x16x4(double a, double b, dbl4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ flt4 mfma16x16x4(float a, float b, flt4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// 16-byte LDS read of an element pair: the tiles are 16-byte aligned with rows
-// of whole 16-byte multiples, so every pair at an even column is (ds_read_b128).
-template <typename S>
-__device__ __forceinline__ typename Vec<S>::V2 lds_pair(const S* p) {
-  return *reinterpret_cast<const typename Vec<S>::V2*>(
-      __builtin_assume_aligned(p, 2 * sizeof(S)));
-}
-
-// Stages one operand tile (ROWS stored rows x BK embedded reduction elements)
-// from global memory into registers and from registers into LDS.
-// UNCHECKED: k-blocks wholly inside the operands skip the per-element checks
-// (measured faster on the large tiles, slower on the small ones).
-template <typename S, bool CPLX, int LAYOUT, int ROWS, int BK, bool UNCHECKED>
-struct TileStage {
-  static constexpr int kPad = kPadOf<S, CPLX>;
-  using V2 = typename Vec<S>::V2;
-  static constexpr int kPairs = ROWS * BK / 2;
-  static constexpr int kPerThread = kPairs / kThreads;
-  static_assert(kPairs % kThreads == 0, "tile does not divide over the workgroup");
-  V2 regs[kPerThread];
-
-  __device__ __forceinline__ static void coords(int pi, int& row, int& qp) {
-    if (LAYOUT == KMajor) {
-      row = pi / (BK / 2);
-      qp = pi % (BK / 2);
-    } else {
-      row = pi % ROWS;
-      qp = pi / ROWS;
-    }
-  }
-
-  // base: operand origin (scalars); ld: leading dimension in elements;
-  // rowBase/rowLimit: stored-row range; q0/qEnd: embedded reduction range.
-  // A k-block wholly inside both ranges is loaded without per-element checks.
-  __device__ __forceinline__ void load(const S* __restrict__ base, int64_t ld, int rowBase,
-                                       int rowLimit, int64_t q0, int64_t qEnd, int tid) {
-    if (UNCHECKED && rowBase + ROWS <= rowLimit && q0 + BK <= qEnd) {
-#pragma unroll
-      for (int u = 0; u < kPerThread; ++u) {
-        int row, qp;
-        coords(tid + u * kThreads, row, qp);
-        const int grow = rowBase + row;
-        const int64_t q = q0 + 2 * qp;
-        if (LAYOUT == KMajor) {
-          const S* p = base + static_cast<int64_t>(grow) * ld * (CPLX ? 2 : 1) + q;
-          regs[u] = V2{p[0], p[1]};
-        } else if (CPLX) {
-          const S* p = base + ((q >> 1) * ld + grow) * 2;
-          regs[u] = V2{p[0], p[1]};
-        } else {
-          regs[u] = V2{base[q * ld + grow], base[(q + 1) * ld + grow]};
-        }
-      }
-      return;
-    }
-#pragma unroll
-    for (int u = 0; u < kPerThread; ++u) {
-      int row, qp;
-      coords(tid + u * kThreads, row, qp);
-      const int grow = rowBase + row;
-      const int64_t q = q0 + 2 * qp;
-      S d0 = S(0), d1 = S(0);
-      if (grow < rowLimit) {
-        if (LAYOUT == KMajor) {
-          const S* p = base + static_cast<int64_t>(grow) * ld * (CPLX ? 2 : 1) + q;
-          if (q < qEnd) d0 = p[0];
-          if (q + 1 < qEnd) d1 = p[1];
-        } else if (CPLX) {
-          if (q < qEnd) {
-            const S* p = base + ((q >> 1) * ld + grow) * 2;
-            d0 = p[0];
-            d1 = p[1];
-          }
-        } else {
-          if (q < qEnd) d0 = base[q * ld + grow];
-          if (q + 1 < qEnd) d1 = base[(q + 1) * ld + grow];
-        }
-      }
-      regs[u] = V2{d0, d1};
-    }
-  }
-
-  __device__ __forceinline__ void store(S (*lds)[BK + kPad], int tid) const {
-#pragma unroll
-    for (int u = 0; u < kPerThread; ++u) {
-      int row, qp;
-      coords(tid + u * kThreads, row, qp);
-      *reinterpret_cast<V2*>(&lds[row][2 * qp]) = regs[u];
-    }
-  }
-};
-
-// Operands of one tile product (element rows m / columns n of C).
+// One operand of one tile product: element (row, l) at X + row * ld + l
+// (K-major) or X + l * ld + row (MN-major).
 template <typename S>
 struct TileOperands {
   const S* A;
   const S* B;
-  int64_t lda, ldb;
-  int m, n;
-  int conjA, conjB;
+  int64_t lda, ldb;  // elements
+  int m, n;          // element rows / columns of C
 };
 
-// LDS of one tile: two buffers of AR stored A rows and BN B rows of BK elements.
-// Rows are whole 16-byte multiples; the 16-byte alignment lets the fragment
-// reads compile to ds_read_b128.
-template <typename S, bool CPLX, int AR, int BN, int BK>
-struct TileSmem {
-  alignas(16) S lA[2][AR][BK + kPadOf<S, CPLX>];
-  alignas(16) S lB[2][BN][BK + kPadOf<S, CPLX>];
-};
+// Moves ROWS rows x one k-block of an operand from global memory through
+// registers to LDS.
+// WIDE: rows (K-major) or reduction indices (MN-major) so far apart that 32-bit
+// lane offsets do not reach over a wave's pieces (tile_wide of gemm_desc.hpp); 64-bit lane
+// addresses, made for every k-block.
+template <typename S, bool CPLX, int LAYOUT, int ROWS, bool WIDE>
+struct TileStage {
+  static constexpr int kComps = CPLX ? 2 : 1;
+  static constexpr int kElem = sizeof(S) * kComps;          // bytes of an element
+  static constexpr int kPerChunk = kChunk / kElem;          // elements of a chunk
+  static constexpr int kBK = kBlockBytes / kElem;           // elements of a k-block
+  static constexpr int kBytes = ROWS * (LAYOUT == KMajor ? kRowBytes : kBlockBytes);
+  // K-major: 16-byte chunks, eight lanes per row; MN-major: single elements,
+  // neighbouring lanes on neighbouring rows
+  static constexpr int kScalars = LAYOUT == KMajor ? kChunk / sizeof(S) : (CPLX ? 2 : 1);
+  static constexpr int kPieceBytes = kScalars * sizeof(S);
+  static constexpr int kPieces = ROWS * kBlockBytes / (kThreads * kPieceBytes);
+  static_assert(kPieces >= 1, "tile smaller than one piece per thread");
+  using Piece = typename VecOf<S, kScalars>::type;
+  struct Regs {
+    Piece p[kPieces];
+  };
 
-// One BM x BN tile of the embedded product over the embedded reduction range
-// [kBegin, kEnd), accumulated in registers. Shared by the single-product
-// kernels and the batched kernels. On return every thread has passed the final
-// barrier, so the LDS buffers may be reused at once (reads that one schedule
-// issues after that barrier only fill registers that are discarded).
-// LEAN: for callers that keep more state live across tiles (the persistent
-// batched kernel), which only take the schedules with one fragment set and one
-// barrier per k-block.
-template <typename S, bool CPLX, int LA, int LB, int WM, int WN, int WAVES_M, int BK,
-          bool LEAN = false>
-struct TileMma {
-  using V2 = typename Vec<S>::V2;
-  using Acc = typename Vec<S>::V4;
-  static constexpr int WAVES_N = 4 / WAVES_M;
-  static constexpr int BM = WM * WAVES_M;
-  static constexpr int BN = WN * WAVES_N;
-  static constexpr int AR = CPLX ? BM / 2 : BM;
-  static constexpr int FM = WM / 16;
-  static constexpr int FN = WN / 16;
-  static_assert(BK % 8 == 0, "k-block must hold whole 8-element sub-blocks");
-  static constexpr bool kF64 = sizeof(S) == 8;
+  // One wave-uniform base per wave and 32-bit lane offsets. K-major: wave w moves
+  // rows w ROWS / 4 .. (w + 1) ROWS / 4 - 1, piece u its rows 8 u .. 8 u + 7 (an
+  // offset per piece); MN-major: the same rows in every piece, piece u
+  // u * pieceStep bytes further on.
+  static constexpr int kWaveRows = ROWS / 4;
+  static constexpr int kOffs = LAYOUT == KMajor ? kPieces : 1;
+  const char* origin;   // the tile's first row, first reduction index
+  const char* base;     // the wave's first row or reduction index
+  int last;             // last row that exists, relative to the tile
+  int64_t rowBytes;
+  int64_t blockStep;    // bytes from one k-block to the next
+  uint32_t pieceStep;
+  uint32_t off[kOffs];
+  int64_t kEnd;         // reduction range in elements, relative to k-block 0
+  int fast;             // k-blocks 0 .. fast - 1 are whole
 
-  // Complex fragment row r (= lane % 16 of the A operand): its complex row
-  // inside the fragment and whether it is an imaginary row.
-  __device__ __forceinline__ static int cplx_row(int r) { return kF64 ? (r & 7) : (r >> 1); }
-  __device__ __forceinline__ static bool imag_row(int r) { return kF64 ? r >= 8 : (r & 1) != 0; }
+  // Row (relative to the tile) of the thread's piece u.
+  __device__ __forceinline__ static int tile_row(int tid, int u) {
+    return LAYOUT == KMajor ? (tid >> 6) * kWaveRows + 8 * u + ((tid & 63) >> 3) : tid % ROWS;
+  }
+  // Reduction index (relative to k-block 0) of the first element of piece u of k-block kb.
+  __device__ __forceinline__ static int64_t first_index(int tid, int u, int kb) {
+    return static_cast<int64_t>(kb) * kBK +
+           (LAYOUT == KMajor ? kPerChunk * (tid & 7) : (tid + kThreads * u) / ROWS);
+  }
 
-  static constexpr int kPad = kPadOf<S, CPLX>;
-  using Smem = TileSmem<S, CPLX, AR, BN, BK>;
-
-  __device__ __forceinline__ static void run(const TileOperands<S>& op, int row0, int col0,
-                                             int64_t kBegin, int64_t kEnd, Smem& sm,
-                                             Acc (&acc)[FM][FN]) {
-    const int arow0 = CPLX ? row0 / 2 : row0;
-    const int nk = static_cast<int>((kEnd - kBegin + BK - 1) / BK);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wid = tid >> 6;
-    const int wm = wid % WAVES_M;
-    const int wn = wid / WAVES_M;
-    const int l16 = lane & 15;
-    const int kk = lane >> 4;
-
-    // Lane-constant complex operand selection (see gemm_desc.hpp):
-    //   real row (t = 0): step0 <- Re(a), step1 <- Im(a) * (conjA == conjB ? -1 : 1)
-    //   imag row (t = 1): step0 <- Im(a) * (conjA ? -1 : 1), step1 <- Re(a) * (conjB ? -1 : 1)
-    // Fragment row r = lane % 16 is an imaginary row when imag_row(r).
-    bool swapPair = false;
-    uint32_t sgn0 = 0, sgn1 = 0;
-    if (CPLX) {
-      swapPair = imag_row(l16);
-      if (!swapPair) {
-        sgn1 = (op.conjA == op.conjB) ? 0x80000000u : 0u;
-      } else {
-        sgn0 = op.conjA ? 0x80000000u : 0u;
-        sgn1 = op.conjB ? 0x80000000u : 0u;
-      }
+  // rows [rowBase, limit) of the operand at X exist (at least one); reduction
+  // elements [k0, k1).
+  __device__ __forceinline__ void init(const S* X, int64_t ld, int rowBase, int limit, int64_t k0,
+                                       int64_t k1) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    last = limit - 1 - rowBase;
+    const int64_t ldBytes = ld * kElem;
+    const uint32_t ld32 = static_cast<uint32_t>(ldBytes);
+    const char* x = reinterpret_cast<const char*>(X) + static_cast<int64_t>(rowBase) *
+                                                           (LAYOUT == KMajor ? ldBytes : kElem);
+    kEnd = k1 - k0;
+    rowBytes = LAYOUT == KMajor ? ldBytes : kElem;
+    origin = x + k0 * (LAYOUT == KMajor ? kElem : ldBytes);
+    if (LAYOUT == KMajor) {
+      const int first = min(wave * kWaveRows, last);
+      base = origin + first * ldBytes;
+      blockStep = kBlockBytes;
+      pieceStep = 0;
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u)
+        off[u % kOffs] = static_cast<uint32_t>(min(tile_row(threadIdx.x, u), last) - first) * ld32 +
+                         kChunk * (lane & 7);
+    } else {
+      constexpr int kPerWave = ROWS < 64 ? 64 / ROWS : 1;  // reduction indices of a wave's piece
+      const int first = ROWS < 64 ? wave * kPerWave : wave * 64 / ROWS;
+      base = origin + first * ldBytes;
+      blockStep = kBK * ldBytes;
+      pieceStep = (kThreads / ROWS) * ld32;
+      off[0] = static_cast<uint32_t>(min(tile_row(threadIdx.x, 0), last)) * kElem;
+      if (ROWS < 64) off[0] += static_cast<uint32_t>(lane / ROWS) * ld32;
     }
+    fast = WIDE ? 0 : static_cast<int>(kEnd / kBK);
+  }
 
-#pragma unroll
-    for (int f = 0; f < FM; ++f)
-#pragma unroll
-      for (int g = 0; g < FN; ++g) acc[f][g] = Acc{S(0), S(0), S(0), S(0)};
+  // readfirstlane: wave-uniform already, but kept in scalar registers for certain
+  __device__ __forceinline__ static __amdgpu_buffer_rsrc_t resource(const char* p) {
+    const uint64_t b = reinterpret_cast<uint64_t>(p);
+    const uint64_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b));
+    const uint64_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<void*>(hi << 32 | (lo & 0xffffffffu)), 0, 0xffffffff, 0x00020000);
+  }
 
-    constexpr bool kUnchecked = WM * WN >= 64 * 64;
-    TileStage<S, CPLX, LA, AR, BK, kUnchecked> stA;
-    TileStage<S, CPLX, LB, BN, BK, kUnchecked> stB;
-
-    // Large tiles: the next 8-element sub-block's fragments are read from LDS while
-    // the current one's MFMAs run (two register sets; 2.6 % faster on the complex
-    // FP64 A^H B tiles with one barrier per k-block, but 6 % slower on FP32 and 0.5 %
-    // on the small ring-step tiles). With the split-barrier schedule below the 64 x 64
-    // wave tiles gain more: FP64 MN-major A (A B) takes it on complex tiles only
-    // (pzgemm_sbs 100000 x 4096 x 4096 63.6 -> 66.6 TFLOP/s; the real ones spill);
-    // FP32 in every layout but real MN-major B, at two waves per SIMD (2048 x 2048 x
-    // 1e5: complex A^H B 110.7 -> 120.3 TFLOP/s, real A^T B 111.6 -> 121.5, real A B
-    // 103.4 -> 118.5; three waves per SIMD, 168 VGPRs: 109.6). Real tiles with
-    // MN-major B read just in time: with the second set they spilled 132 VGPRs in
-    // FP64 (2048 x 2048 x 1e5 A^T B^T 44.7 TFLOP/s, 59.6 without).
-    constexpr bool kPrefetch =
-        (kF64 && WM * WN >= 64 * 64 && (CPLX || LB == KMajor) &&
-         (LA == KMajor || (!LEAN && CPLX && WM * WN == 64 * 64))) ||
-        (!kF64 && !LEAN && BK == 16 && WM * WN == 64 * 64 && (CPLX || LB == KMajor));
-    if constexpr (kPrefetch) {
-      static_assert((BK / 8) % 2 == 0, "sub-blocks alternate between two register sets");
-      S a0[2][FM], a1[2][FM];
-      V2 b[2][FN];
-      auto read_frags = [&](int set, int buf, int kb8) {
+  // k-block kb < fast. Buffer loads: the base is four scalar registers, the lane
+  // offset one vector register that never changes.
+  __device__ __forceinline__ void load_fast(Regs& r, int kb) const {
+    const __amdgpu_buffer_rsrc_t rsrc = resource(base + kb * blockStep);
 #pragma unroll
-        for (int f = 0; f < FM; ++f) {
-          const int sr = CPLX ? (wm * WM) / 2 + 8 * f + cplx_row(l16) : wm * WM + 16 * f + l16;
-          const V2 v = lds_pair(&sm.lA[buf][sr][kb8 * 8 + 2 * kk]);
-          if (CPLX) {
-            const S x = swapPair ? v.y : v.x;
-            const S y = swapPair ? v.x : v.y;
-            a0[set][f] = flip_sign(x, sgn0);
-            a1[set][f] = flip_sign(y, sgn1);
-          } else {
-            a0[set][f] = v.x;
-            a1[set][f] = v.y;
-          }
+    for (int u = 0; u < kPieces; ++u)
+      r.p[u] = buffer_load<Piece>(
+          rsrc, off[u % kOffs],
+          LAYOUT == KMajor ? 0 : __builtin_amdgcn_readfirstlane(u * pieceStep));
+  }
+
+  // k-block kb, whole or not. Reduction indices past the range are zero in both
+  // operands; they are read from the range's last element, so that every load is
+  // issued without a branch. A k-block past the range leaves r as it is.
+  __device__ __forceinline__ void load(Regs& r, int kb) const {
+    if (!WIDE && kb < fast) return load_fast(r, kb);
+    const int64_t left = kEnd - static_cast<int64_t>(kb) * kBK;
+    if (left <= 0) return;
+    const int rem = static_cast<int>(min(left, static_cast<int64_t>(kBK)));
+    // The thread index passes through an empty statement so that these offsets
+    // are made here, once, and not kept in registers through the loop.
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    using Elem = typename VecOf<S, CPLX ? 2 : 1>::type;
+    constexpr int kElems = kPieceBytes / kElem;  // of one piece, along the reduction index
+    const int64_t ldBytes = blockStep / kBK;     // MN-major
+    const char* b = LAYOUT == KMajor ? base + kb * blockStep : origin + kb * blockStep;
+    const __amdgpu_buffer_rsrc_t rsrc = resource(b);
+    bool in[kPieces][kElems];
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u)
+#pragma unroll
+      for (int e = 0; e < kElems; ++e) {
+        const int first = LAYOUT == KMajor ? kPerChunk * (tid & 7) : (tid + kThreads * u) / ROWS;
+        in[u][e] = first + e < rem;
+        const int l = min(first + e, rem - 1);
+        Elem v;
+        if constexpr (WIDE) {
+          using Loose = typename VecOf<S, CPLX ? 2 : 1>::loose;
+          const int64_t row = min(tile_row(tid, u), last);
+          v = *reinterpret_cast<const Loose*>(
+              LAYOUT == KMajor ? origin + row * rowBytes + kb * blockStep + l * kElem
+                               : b + l * ldBytes + row * kElem);
+        } else if constexpr (LAYOUT == KMajor) {
+          v = buffer_load<Elem>(rsrc, off[u] + (l - first) * kElem, 0);
+        } else {
+          v = buffer_load<Elem>(rsrc,
+                                min(tile_row(tid, u), last) * kElem +
+                                    static_cast<uint32_t>(l) * static_cast<uint32_t>(ldBytes),
+                                0);
         }
-#pragma unroll
-        for (int g = 0; g < FN; ++g) {
-          const int j = wn * WN + 16 * g + l16;
-          b[set][g] = lds_pair(&sm.lB[buf][j][kb8 * 8 + 2 * kk]);
+        if constexpr (kScalars == 1) {
+          r.p[u] = v;
+        } else if constexpr (CPLX) {
+          r.p[u][2 * e] = v[0];
+          r.p[u][2 * e + 1] = v[1];
+        } else {
+          r.p[u][e] = v;
         }
-      };
-
-      // half = 0: the even reduction elements of a sub-block, 1: the odd ones
-      auto mfma_half = [&](int set, int half) {
-#pragma unroll
-        for (int f = 0; f < FM; ++f)
-#pragma unroll
-          for (int g = 0; g < FN; ++g)
-            acc[f][g] = half ? mfma16x16x4(a1[set][f], b[set][g].y, acc[f][g])
-                             : mfma16x16x4(a0[set][f], b[set][g].x, acc[f][g]);
-      };
-
-      if (nk > 0) {
-        stA.load(op.A, op.lda, arow0, op.m, kBegin, kEnd, tid);
-        stB.load(op.B, op.ldb, col0, op.n, kBegin, kEnd, tid);
-        stA.store(sm.lA[0], tid);
-        stB.store(sm.lB[0], tid);
       }
-      __syncthreads();
-      if (nk > 0) read_frags(0, 0, 0);
+    if (rem == kBK) return;
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u)
+#pragma unroll
+      for (int e = 0; e < kElems; ++e) {
+        if constexpr (kScalars == 1) {
+          r.p[u] = in[u][e] ? r.p[u] : S(0);
+        } else {
+#pragma unroll
+          for (int c = 0; c < kComps; ++c)
+            r.p[u][kComps * e + c] = in[u][e] ? r.p[u][kComps * e + c] : S(0);
+        }
+      }
+  }
 
-      // 64 x 64 wave tiles (two waves per SIMD) except real MN-major B, whose staging
-      // leaves no registers for it; the 128 x 64 tiles spill with it.
-      constexpr bool kSplitBarrier =
-          !LEAN && BK == 16 && WM * WN == 64 * 64 && (CPLX || LB == KMajor);
-      if constexpr (kSplitBarrier) {
-        // A k-block's 4 FM FN MFMAs in quarters: (sub-block 0, even elements) with the
-        // reads of sub-block 1; the staged stores into the other buffer; (sub-block 0,
-        // odd), which covers the stores' completion; the barrier; the next k-block's
-        // sub-block 0 reads; both quarters of sub-block 1, which cover those reads.
-        // Against one barrier after all the MFMAs of a k-block, with the stores and
-        // reads on either side of it: 2048 x 2048 x 2e5 complex A^H B 109.8 -> 102.7 ms.
-        if (nk > 1) {
-          stA.load(op.A, op.lda, arow0, op.m, kBegin + BK, kEnd, tid);
-          stB.load(op.B, op.ldb, col0, op.n, kBegin + BK, kEnd, tid);
-        }
-        // k-block it + 2 into the staging registers once they are stored. Real tiles
-        // (eight staged pairs per thread) issue these loads right after the stores;
-        // complex tiles (six) after the barrier and the next fragment reads, which
-        // measured 1-2 % faster for each.
-        // The stores and the reads after the barrier are unconditional (branches here
-        // make the wait counts conservative): in the last k-block they store the
-        // staged registers' last k-block once more into the buffer that is no longer
-        // read, and read them back into registers that are not used (reads issued
-        // after the final barrier whose values are discarded).
-        for (int it = 0; it < nk; ++it) {
-          const int cur = it & 1;
-          read_frags(1, cur, 1);
-          mfma_half(0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-          stA.store(sm.lA[cur ^ 1], tid);
-          stB.store(sm.lB[cur ^ 1], tid);
-          if constexpr (!CPLX) {
-            if (it + 2 < nk) {
-              const int64_t q0 = kBegin + static_cast<int64_t>(it + 2) * BK;
-              stA.load(op.A, op.lda, arow0, op.m, q0, kEnd, tid);
-              stB.load(op.B, op.ldb, col0, op.n, q0, kEnd, tid);
-            }
-          }
-          mfma_half(0, 1);
-          __builtin_amdgcn_sched_barrier(0);  // these MFMAs cover the stores' completion
-          __syncthreads();
-          read_frags(0, cur ^ 1, 0);
-          if constexpr (CPLX) {
-            if (it + 2 < nk) {
-              const int64_t q0 = kBegin + static_cast<int64_t>(it + 2) * BK;
-              stA.load(op.A, op.lda, arow0, op.m, q0, kEnd, tid);
-              stB.load(op.B, op.ldb, col0, op.n, q0, kEnd, tid);
-            }
-          }
-          mfma_half(1, 0);
-          mfma_half(1, 1);
-        }
-        return;
-      }
+  __device__ __forceinline__ static void store(const Regs& r, unsigned char* lds) {
+    unsigned char* p = LAYOUT == KMajor
+                           ? lds + tile_row(threadIdx.x, 0) * kRowBytes + kChunk * (threadIdx.x & 7)
+                           : lds + threadIdx.x * kElem;
+    constexpr int kStep = LAYOUT == KMajor ? 8 * kRowBytes : kThreads * kElem;
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) *reinterpret_cast<Piece*>(p + u * kStep) = r.p[u];
+  }
+};
 
-      for (int it = 0; it < nk; ++it) {
-        const int cur = it & 1;
-        const bool more = it + 1 < nk;
-        if (more) {
-          const int64_t q0 = kBegin + static_cast<int64_t>(it + 1) * BK;
-          stA.load(op.A, op.lda, arow0, op.m, q0, kEnd, tid);
-          stB.load(op.B, op.ldb, col0, op.n, q0, kEnd, tid);
-        }
+// Fragments of one operand for one sub-block: F fragments of 16 rows.
+template <typename S, bool CPLX, int LAYOUT, int ROWS, int F>
+struct TileFrags {
+  using Stage = TileStage<S, CPLX, LAYOUT, ROWS, false>;
+  static constexpr int kSteps = Stage::kPerChunk;  // MFMA steps of a sub-block
+  // MN-major: neighbouring rows of one read, each a fragment of its own
+  static constexpr int VR = LAYOUT == KMajor ? 1 : (kSteps < F ? kSteps : F);
+  static_assert(F % VR == 0, "fragments come in groups of VR");
+  S re[kSteps][F];
+  S im[CPLX ? kSteps : 1][F];
 
-#pragma unroll
-        for (int kb8 = 0; kb8 < BK / 8; ++kb8) {
-          const int s = kb8 & 1;
-          if (kb8 + 1 < BK / 8) read_frags(s ^ 1, cur, kb8 + 1);
-#pragma unroll
-          for (int f = 0; f < FM; ++f)
-#pragma unroll
-            for (int g = 0; g < FN; ++g) acc[f][g] = mfma16x16x4(a0[s][f], b[s][g].x, acc[f][g]);
-#pragma unroll
-          for (int f = 0; f < FM; ++f)
-#pragma unroll
-            for (int g = 0; g < FN; ++g) acc[f][g] = mfma16x16x4(a1[s][f], b[s][g].y, acc[f][g]);
-        }
+  // row (relative to the wave) of entry i of fragment f
+  __device__ __forceinline__ static int row(int f, int i) {
+    return 16 * VR * (f / VR) + VR * i + f % VR;
+  }
 
-        if (more) {
-          stA.store(sm.lA[cur ^ 1], tid);
-          stB.store(sm.lB[cur ^ 1], tid);
+  __device__ __forceinline__ void read(const unsigned char* lds, int waveRow, int sub) {
+    const int l16 = threadIdx.x & 15;
+    const int kk = (threadIdx.x & 63) >> 4;
+    if constexpr (LAYOUT == KMajor) {
+      constexpr int kN = kChunk / sizeof(S);
+      using V = typename VecOf<S, kN>::type;
+      const unsigned char* p = lds + (waveRow + l16) * kRowBytes + kChunk * kk;
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+        const V v = *reinterpret_cast<const V*>(p + f * 16 * kRowBytes + sub * 4 * kChunk);
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+          re[s][f] = v[CPLX ? 2 * s : s];
+          if (CPLX) im[s % (CPLX ? kSteps : 1)][f] = v[(CPLX ? 2 * s + 1 : s)];
         }
-        __syncthreads();
-        if (more) read_frags(0, cur ^ 1, 0);  // the next k-block's first sub-block
-      }
-    } else if constexpr (WM * WN < 64 * 64 && (CPLX || LA != MNMajor || LB != MNMajor)) {
-      // Small tiles (small m, n; HBM-bound with a long reduction): the global loads
-      // run two k-blocks ahead through two register sets, so each workgroup keeps
-      // twice the bytes in flight; fragments are read just in time. The real
-      // MN-major x MN-major variant stays one ahead: in FP64 the second set takes it
-      // past 128 VGPRs, one resident workgroup fewer per CU, and it ran 7 % slower.
-      TileStage<S, CPLX, LA, AR, BK, kUnchecked> stA2;
-      TileStage<S, CPLX, LB, BN, BK, kUnchecked> stB2;
-      if (nk > 0) {
-        stA.load(op.A, op.lda, arow0, op.m, kBegin, kEnd, tid);
-        stB.load(op.B, op.ldb, col0, op.n, kBegin, kEnd, tid);
-        stA.store(sm.lA[0], tid);
-        stB.store(sm.lB[0], tid);
-      }
-      if (nk > 1) {
-        stA2.load(op.A, op.lda, arow0, op.m, kBegin + BK, kEnd, tid);
-        stB2.load(op.B, op.ldb, col0, op.n, kBegin + BK, kEnd, tid);
-      }
-      __syncthreads();
-      if constexpr (kF64 && BK == 16 && !LEAN) {
-        // The split-barrier schedule of the large tiles with the loads two ahead:
-        // fragments in two register sets (sub-block 1's read during sub-block 0's
-        // MFMAs, the next k-block's sub-block 0 right after the barrier), the staged
-        // stores between the two halves of sub-block 0's MFMAs, sub-block 1's after
-        // the barrier. Stores and post-barrier reads are unconditional as there; a
-        // staging set never loaded (one k-block) stores zeros.
-        S fa0[2][FM], fa1[2][FM];
-        V2 fb[2][FN];
-        auto rd = [&](int set, int buf, int kb8) {
-#pragma unroll
-          for (int f = 0; f < FM; ++f) {
-            const int sr = CPLX ? (wm * WM) / 2 + 8 * f + cplx_row(l16) : wm * WM + 16 * f + l16;
-            const V2 v = lds_pair(&sm.lA[buf][sr][kb8 * 8 + 2 * kk]);
-            if (CPLX) {
-              const S x = swapPair ? v.y : v.x;
-              const S y = swapPair ? v.x : v.y;
-              fa0[set][f] = flip_sign(x, sgn0);
-              fa1[set][f] = flip_sign(y, sgn1);
-            } else {
-              fa0[set][f] = v.x;
-              fa1[set][f] = v.y;
-            }
-          }
-#pragma unroll
-          for (int g = 0; g < FN; ++g) {
-            const int j = wn * WN + 16 * g + l16;
-            fb[set][g] = lds_pair(&sm.lB[buf][j][kb8 * 8 + 2 * kk]);
-          }
-        };
-        auto mm = [&](int set, int half) {
-#pragma unroll
-          for (int f = 0; f < FM; ++f)
-#pragma unroll
-            for (int g = 0; g < FN; ++g)
-              acc[f][g] = half ? mfma16x16x4(fa1[set][f], fb[set][g].y, acc[f][g])
-                               : mfma16x16x4(fa0[set][f], fb[set][g].x, acc[f][g]);
-        };
-        if (nk == 1) {
-#pragma unroll
-          for (int u = 0; u < decltype(stA2)::kPerThread; ++u) stA2.regs[u] = V2{S(0), S(0)};
-#pragma unroll
-          for (int u = 0; u < decltype(stB2)::kPerThread; ++u) stB2.regs[u] = V2{S(0), S(0)};
-        }
-        if (nk > 0) rd(0, 0, 0);
-        auto kblock2 = [&](int it, auto& la, auto& lb, const auto& sa, const auto& sb) {
-          const int cur = it & 1;
-          if (it + 2 < nk) {
-            const int64_t q0 = kBegin + static_cast<int64_t>(it + 2) * BK;
-            la.load(op.A, op.lda, arow0, op.m, q0, kEnd, tid);
-            lb.load(op.B, op.ldb, col0, op.n, q0, kEnd, tid);
-          }
-          rd(1, cur, 1);
-          mm(0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-          sa.store(sm.lA[cur ^ 1], tid);
-          sb.store(sm.lB[cur ^ 1], tid);
-          mm(0, 1);
-          __builtin_amdgcn_sched_barrier(0);
-          __syncthreads();
-          rd(0, cur ^ 1, 0);
-          mm(1, 0);
-          mm(1, 1);
-        };
-        for (int it = 0; it < nk; it += 2) {
-          kblock2(it, stA, stB, stA2, stB2);
-          if (it + 1 < nk) kblock2(it + 1, stA2, stB2, stA, stB);
-        }
-        return;
-      }
-      // one k-block: (la, lb) receive k-block it + 2, (sa, sb) hold it + 1
-      auto kblock = [&](int it, auto& la, auto& lb, const auto& sa, const auto& sb) {
-        const int cur = it & 1;
-        if (it + 2 < nk) {
-          const int64_t q0 = kBegin + static_cast<int64_t>(it + 2) * BK;
-          la.load(op.A, op.lda, arow0, op.m, q0, kEnd, tid);
-          lb.load(op.B, op.ldb, col0, op.n, q0, kEnd, tid);
-        }
-#pragma unroll
-        for (int kb8 = 0; kb8 < BK / 8; ++kb8) {
-          S a0[FM], a1[FM];
-          V2 b[FN];
-#pragma unroll
-          for (int f = 0; f < FM; ++f) {
-            const int sr = CPLX ? (wm * WM) / 2 + 8 * f + cplx_row(l16) : wm * WM + 16 * f + l16;
-            const V2 v = lds_pair(&sm.lA[cur][sr][kb8 * 8 + 2 * kk]);
-            if (CPLX) {
-              const S x = swapPair ? v.y : v.x;
-              const S y = swapPair ? v.x : v.y;
-              a0[f] = flip_sign(x, sgn0);
-              a1[f] = flip_sign(y, sgn1);
-            } else {
-              a0[f] = v.x;
-              a1[f] = v.y;
-            }
-          }
-#pragma unroll
-          for (int g = 0; g < FN; ++g) {
-            const int j = wn * WN + 16 * g + l16;
-            b[g] = lds_pair(&sm.lB[cur][j][kb8 * 8 + 2 * kk]);
-          }
-#pragma unroll
-          for (int f = 0; f < FM; ++f)
-#pragma unroll
-            for (int g = 0; g < FN; ++g) acc[f][g] = mfma16x16x4(a0[f], b[g].x, acc[f][g]);
-#pragma unroll
-          for (int f = 0; f < FM; ++f)
-#pragma unroll
-            for (int g = 0; g < FN; ++g) acc[f][g] = mfma16x16x4(a1[f], b[g].y, acc[f][g]);
-        }
-        if (it + 1 < nk) {
-          sa.store(sm.lA[cur ^ 1], tid);
-          sb.store(sm.lB[cur ^ 1], tid);
-        }
-        __syncthreads();
-      };
-      for (int it = 0; it < nk; it += 2) {
-        kblock(it, stA, stB, stA2, stB2);
-        if (it + 1 < nk) kblock(it + 1, stA2, stB2, stA, stB);
       }
     } else {
-      // each sub-block's fragments are read right before its MFMAs
-      if (nk > 0) {
-        stA.load(op.A, op.lda, arow0, op.m, kBegin, kEnd, tid);
-        stB.load(op.B, op.ldb, col0, op.n, kBegin, kEnd, tid);
-        stA.store(sm.lA[0], tid);
-        stB.store(sm.lB[0], tid);
-      }
-      __syncthreads();
-
-      for (int it = 0; it < nk; ++it) {
-        const int cur = it & 1;
-        const bool more = it + 1 < nk;
-        if (more) {
-          const int64_t q0 = kBegin + static_cast<int64_t>(it + 1) * BK;
-          stA.load(op.A, op.lda, arow0, op.m, q0, kEnd, tid);
-          stB.load(op.B, op.ldb, col0, op.n, q0, kEnd, tid);
-        }
-
+      constexpr int kN = VR * (CPLX ? 2 : 1);
+      using V = typename VecOf<S, kN>::type;
+      const unsigned char* p =
+          lds + (kSteps * kk * ROWS + waveRow + VR * l16) * Stage::kElem;
 #pragma unroll
-        for (int kb8 = 0; kb8 < BK / 8; ++kb8) {
-          S a0[FM], a1[FM];
-          V2 b[FN];
+      for (int s = 0; s < kSteps; ++s)
 #pragma unroll
-          for (int f = 0; f < FM; ++f) {
-            const int sr = CPLX ? (wm * WM) / 2 + 8 * f + cplx_row(l16) : wm * WM + 16 * f + l16;
-            const V2 v = lds_pair(&sm.lA[cur][sr][kb8 * 8 + 2 * kk]);
-            if (CPLX) {
-              const S x = swapPair ? v.y : v.x;
-              const S y = swapPair ? v.x : v.y;
-              a0[f] = flip_sign(x, sgn0);
-              a1[f] = flip_sign(y, sgn1);
-            } else {
-              a0[f] = v.x;
-              a1[f] = v.y;
+        for (int q = 0; q < F / VR; ++q) {
+          const V v = *reinterpret_cast<const V*>(
+              p + ((sub * (Stage::kBK / 2) + s) * ROWS + 16 * VR * q) * Stage::kElem);
+          if constexpr (kN == 1) {
+            re[s][q] = v;
+          } else {
+#pragma unroll
+            for (int w = 0; w < VR; ++w) {
+              re[s][VR * q + w] = v[CPLX ? 2 * w : w];
+              if (CPLX) im[s % (CPLX ? kSteps : 1)][VR * q + w] = v[CPLX ? 2 * w + 1 : w];
             }
           }
-#pragma unroll
-          for (int g = 0; g < FN; ++g) {
-            const int j = wn * WN + 16 * g + l16;
-            b[g] = lds_pair(&sm.lB[cur][j][kb8 * 8 + 2 * kk]);
-          }
-#pragma unroll
-          for (int f = 0; f < FM; ++f)
-#pragma unroll
-            for (int g = 0; g < FN; ++g) acc[f][g] = mfma16x16x4(a0[f], b[g].x, acc[f][g]);
-#pragma unroll
-          for (int f = 0; f < FM; ++f)
-#pragma unroll
-            for (int g = 0; g < FN; ++g) acc[f][g] = mfma16x16x4(a1[f], b[g].y, acc[f][g]);
         }
+    }
+  }
+};
 
-        if (more) {
-          stA.store(sm.lA[cur ^ 1], tid);
-          stB.store(sm.lB[cur ^ 1], tid);
+// Tile of AR x BN elements of C (four waves in a 2 x 2 grid, each FM x FN
+// fragments of 16 x 16 elements) over the embedded reduction range
+// [kBegin, kEnd), accumulated in registers. WIDE: see TileStage. CONJ: one of A and B is conjugated
+// (see flip_result). On return every thread has passed the final barrier, so the
+// LDS buffers may be reused at once (reads issued after that barrier only fill
+// registers that are discarded).
+template <typename S, bool CPLX, bool CONJ, int LA, int LB, int FM, int FN, bool WIDE = false>
+struct TileMma {
+  static constexpr int WAVES_M = 2, WAVES_N = 2;
+  static constexpr int AR = 16 * FM * WAVES_M;  // element rows
+  static constexpr int BN = 16 * FN * WAVES_N;
+  static constexpr bool kF64 = sizeof(S) == 8;
+  static constexpr int kComps = CPLX ? 2 : 1;
+  using V4 = typename VecOf<S, 4>::type;
+  using StageA = TileStage<S, CPLX, LA, AR, WIDE>;
+  using StageB = TileStage<S, CPLX, LB, BN, WIDE>;
+  using FragsA = TileFrags<S, CPLX, LA, AR, FM>;
+  using FragsB = TileFrags<S, CPLX, LB, BN, FN>;
+  static constexpr int kSteps = FragsA::kSteps;
+  static constexpr int kPasses = kSteps * (CPLX ? 4 : 1);  // of FM x FN MFMAs per sub-block
+
+  struct Smem {
+    alignas(16) unsigned char a[2][StageA::kBytes];
+    alignas(16) unsigned char b[2][StageB::kBytes];
+  };
+  struct Acc {
+    V4 re[FM][FN];
+    V4 im[CPLX ? FM : 1][CPLX ? FN : 1];
+  };
+
+  // The imaginary part of the sum is to be negated: the kernel computes A B, or
+  // conj(A) B for CONJ, and conj(A) conj(B) = conj(A B), A conj(B) = conj(conj(A) B).
+  __device__ __forceinline__ static bool flip_result(int conjA, int conjB) {
+    return CPLX && (CONJ ? !conjA : (conjA && conjB));
+  }
+
+  // pass p of a sub-block: FM x FN MFMAs
+  __device__ __forceinline__ static void mfma_pass(Acc& acc, const FragsA& a, const FragsB& b,
+                                                   int p) {
+    if constexpr (!CPLX) {
+#pragma unroll
+      for (int f = 0; f < FM; ++f)
+#pragma unroll
+        for (int g = 0; g < FN; ++g)
+          acc.re[f][g] = mfma16x16x4<false>(b.re[p][g], a.re[p][f], acc.re[f][g]);
+    } else {
+      const int s = p / 4;
+#pragma unroll
+      for (int f = 0; f < FM; ++f) {
+        const S ar = a.re[s][f], ai = a.im[s][f];
+        // re += ar br -+ ai bi; im += +-ai br + ar bi
+        const S minus = kF64 ? ai : -ai;
+#pragma unroll
+        for (int g = 0; g < FN; ++g) {
+          if (p % 4 == 0)
+            acc.re[f][g] = mfma16x16x4<false>(b.re[s][g], ar, acc.re[f][g]);
+          else if (p % 4 == 1)
+            acc.re[f][g] =
+                CONJ ? mfma16x16x4<false>(b.im[s][g], ai, acc.re[f][g])
+                     : mfma16x16x4<kF64>(b.im[s][g], minus, acc.re[f][g]);
+          else if (p % 4 == 2)
+            acc.im[f][g] =
+                CONJ ? mfma16x16x4<kF64>(b.re[s][g], minus, acc.im[f][g])
+                     : mfma16x16x4<false>(b.re[s][g], ai, acc.im[f][g]);
+          else
+            acc.im[f][g] = mfma16x16x4<false>(b.im[s][g], ar, acc.im[f][g]);
         }
-        __syncthreads();
       }
     }
   }
 
-  // Calls f(i, j, re, im) for every element of the tile inside m x n.
-  // Accumulators of lane (kk = lane / 16) of column lane % 16: FP64 rows
-  // kk + 4 r, i.e. (re, im) of complex rows kk and kk + 4 in (acc[0], acc[2])
-  // and (acc[1], acc[3]); FP32 rows 4 kk + r, i.e. (re, im) of complex rows
-  // 2 kk and 2 kk + 1 in (acc[0], acc[1]) and (acc[2], acc[3]).
-  template <typename F>
-  __device__ __forceinline__ static void for_each(int row0, int col0, int m, int n,
-                                                  const Acc (&acc)[FM][FN], F&& f) {
-    const int lane = threadIdx.x & 63;
-    const int wid = threadIdx.x >> 6;
-    const int wm = wid % WAVES_M;
-    const int wn = wid / WAVES_M;
-    const int l16 = lane & 15;
-    const int kk = lane >> 4;
-#pragma unroll
-    for (int fm = 0; fm < FM; ++fm) {
-#pragma unroll
-      for (int g = 0; g < FN; ++g) {
-        const int j = col0 + wn * WN + 16 * g + l16;
-        if (j >= n) continue;
-        const Acc v = acc[fm][g];
-        if (CPLX) {
-          const int base = row0 / 2 + (wm * WM) / 2 + 8 * fm;
-          if (kF64) {
-            if (base + kk < m) f(base + kk, j, v[0], v[2]);
-            if (base + kk + 4 < m) f(base + kk + 4, j, v[1], v[3]);
-          } else {
-            if (base + 2 * kk < m) f(base + 2 * kk, j, v[0], v[1]);
-            if (base + 2 * kk + 1 < m) f(base + 2 * kk + 1, j, v[2], v[3]);
-          }
-        } else {
-          const int p0 = row0 + wm * WM + 16 * fm + (kF64 ? kk : 4 * kk);
-          const int step = kF64 ? 4 : 1;
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (p0 + step * r < m) f(p0 + step * r, j, v[r], S(0));
-        }
+  __device__ __forceinline__ static void run(const TileOperands<S>& op, int row0, int col0,
+                                             int64_t kBegin, int64_t kEnd, Smem& sm, Acc& acc) {
+    const int wave = threadIdx.x >> 6;
+    const int wa = (wave % WAVES_M) * 16 * FM;
+    const int wb = (wave / WAVES_M) * 16 * FN;
+    const int64_t k0 = kBegin / kComps, k1 = kEnd / kComps;
+    const int nk = static_cast<int>((k1 - k0 + StageA::kBK - 1) / StageA::kBK);
+    StageA sa;
+    StageB sb;
+    sa.init(op.A, op.lda, row0, op.m, k0, k1);
+    sb.init(op.B, op.ldb, col0, op.n, k0, k1);
+    auto load = [&](typename StageA::Regs& ra, typename StageB::Regs& rb, int kb) {
+      sa.load(ra, kb);
+      sb.load(rb, kb);
+    };
+
+    // Small wave tiles load two k-blocks ahead through two register sets, the
+    // larger ones one and a half (k-block it + 2 as soon as it + 1 is stored).
+    constexpr bool kTwoAhead = FM * FN * kComps <= 4;
+    typename StageA::Regs ra[kTwoAhead ? 2 : 1];
+    typename StageB::Regs rb[kTwoAhead ? 2 : 1];
+    FragsA fa[2];
+    FragsB fb[2];
+    const int whole = min(sa.fast, sb.fast);
+    if (nk > 0) {
+      typename StageA::Regs pa = {};
+      typename StageB::Regs pb = {};
+      constexpr int kSet = kTwoAhead ? 1 : 0;  // register set of k-block 1
+      if (whole >= 2) {  // both in flight together
+        sa.load_fast(pa, 0);
+        sb.load_fast(pb, 0);
+        sa.load_fast(ra[kSet], 1);
+        sb.load_fast(rb[kSet], 1);
+        StageA::store(pa, sm.a[0]);
+        StageB::store(pb, sm.b[0]);
+      } else {
+        load(pa, pb, 0);
+        load(ra[kSet], rb[kSet], 1);
+        StageA::store(pa, sm.a[0]);
+        StageB::store(pb, sm.b[0]);
       }
     }
+#pragma unroll
+    for (int f = 0; f < FM; ++f)
+#pragma unroll
+      for (int g = 0; g < FN; ++g) {
+        acc.re[f][g] = V4{S(0), S(0), S(0), S(0)};
+        if (CPLX) acc.im[f % (CPLX ? FM : 1)][g % (CPLX ? FN : 1)] = V4{S(0), S(0), S(0), S(0)};
+      }
+    if (nk == 0) return;
+    __syncthreads();
+    fa[0].read(sm.a[0], wa, 0);
+    fb[0].read(sm.b[0], wb, 0);
+
+    // One k-block over LDS buffer CUR: sub-block 0's first half with the reads of
+    // sub-block 1; the staged stores into the other buffer; its second half, which
+    // covers the stores' completion; the barrier; the next k-block's sub-block 0
+    // reads; sub-block 1, which covers those reads. The stores and the reads after
+    // the barrier are unconditional (branches make the wait counts conservative):
+    // in the last k-block they store staged registers into the buffer that is no
+    // longer read, and read values that are not used.
+    // next(set): loads k-block it + 2 into register set `set`; tail: these loads
+    // may be partial.
+    auto kblock = [&](auto cur, auto tail, auto next) {
+      constexpr bool kTail = decltype(tail)::value;
+      constexpr int CUR = decltype(cur)::value;
+      constexpr int kStored = kTwoAhead ? CUR ^ 1 : 0;  // register set of k-block it + 1
+      fa[1].read(sm.a[CUR], wa, 1);
+      fb[1].read(sm.b[CUR], wb, 1);
+      if (kTwoAhead) next(CUR);
+#pragma unroll
+      for (int p = 0; p < kPasses / 2; ++p) mfma_pass(acc, fa[0], fb[0], p);
+      __builtin_amdgcn_sched_barrier(0);
+      StageA::store(ra[kStored], sm.a[CUR ^ 1]);
+      StageB::store(rb[kStored], sm.b[CUR ^ 1]);
+      if (!kTwoAhead && !kTail) next(0);
+#pragma unroll
+      for (int p = kPasses / 2; p < kPasses; ++p) mfma_pass(acc, fa[0], fb[0], p);
+      __builtin_amdgcn_sched_barrier(0);  // these MFMAs cover the stores' completion
+      __syncthreads();
+      if (!kTwoAhead && kTail) next(0);  // fewer registers are live here
+      fa[0].read(sm.a[CUR ^ 1], wa, 0);
+      fb[0].read(sm.b[CUR ^ 1], wb, 0);
+#pragma unroll
+      for (int p = 0; p < kPasses; ++p) mfma_pass(acc, fa[1], fb[1], p);
+      __builtin_amdgcn_sched_barrier(0);  // the next k-block's reads stay behind these (registers)
+    };
+    // While both k-blocks that an iteration loads are whole, the loads are
+    // unconditional: the wait counts stay exact (a load that may not be issued
+    // makes every later wait a full one) and the loop holds no branch.
+    int it = 0;
+    for (; it + 3 < whole; it += 2) {
+      auto next = [&](int kb) {
+        return [&, kb](int set) {
+          sa.load_fast(ra[set], kb);
+          sb.load_fast(rb[set], kb);
+        };
+      };
+      kblock(Index<0>(), Index<0>(), next(it + 2));
+      kblock(Index<1>(), Index<0>(), next(it + 3));
+    }
+    auto next = [&](int kb) {
+      return [&, kb](int set) {
+        if (kb < nk) load(ra[set], rb[set], kb);
+      };
+    };
+    for (; it < nk; it += 2) {
+      kblock(Index<0>(), Index<1>(), next(it + 2));
+      if (it + 1 < nk) kblock(Index<1>(), Index<1>(), next(it + 3));
+    }
+  }
+
+  // Calls f(i, j, re, im) for every element of the tile inside m x n; `flip`:
+  // see flip_result.
+  template <typename F>
+  __device__ __forceinline__ static void for_each(int row0, int col0, int m, int n, bool flip,
+                                                  const Acc& acc, F&& f) {
+    const int wave = threadIdx.x >> 6;
+    const int l16 = threadIdx.x & 15;
+    const int kk = (threadIdx.x & 63) >> 4;
+    const int wr = row0 + (wave % WAVES_M) * 16 * FM;
+    const int wc = col0 + (wave / WAVES_M) * 16 * FN;
+#pragma unroll
+    for (int g = 0; g < FN; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = wc + FragsB::row(g, kF64 ? kk + 4 * r : 4 * kk + r);
+        if (j >= n) continue;
+#pragma unroll
+        for (int fm = 0; fm < FM; ++fm) {
+          const int i = wr + FragsA::row(fm, l16);
+          if (i >= m) continue;
+          S im = S(0);
+          if (CPLX) {
+            im = acc.im[fm % (CPLX ? FM : 1)][g % (CPLX ? FN : 1)][r];
+            im = flip ? -im : im;
+          }
+          f(i, j, acc.re[fm][g][r], im);
+        }
+      }
   }
 };
 
@@ -637,6 +596,12 @@ __device__ __forceinline__ void store_work(S* w, int64_t Mp, int i, int j, S re,
   S* p = w + static_cast<int64_t>(j) * Mp + (CPLX ? 2 * i : i);
   p[0] = re;
   if (CPLX) p[1] = im;
+}
+
+__device__ __forceinline__ double flip_sign(double x, uint32_t hiMask) {
+  uint64_t b = __builtin_bit_cast(uint64_t, x);
+  b ^= static_cast<uint64_t>(hiMask) << 32;
+  return __builtin_bit_cast(double, b);
 }
 
 }  // namespace tile

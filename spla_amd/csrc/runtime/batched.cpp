@@ -195,8 +195,13 @@ void GroupedLaunch::build(spla::ContextInternal& ctx, bool complex, SplaOperatio
   desc_.betaZero = (desc_.betaRe == 0.0 && desc_.betaIm == 0.0) ? 1 : 0;
   desc_.conjA = (complex && opA == SPLA_OP_CONJ_TRANSPOSE) ? 1 : 0;
   desc_.conjB = 0;
-  kernels_ = batched_kernels(complex, opA == SPLA_OP_NONE ? MNMajor : KMajor, sched.cfg,
-                             persistent);
+  bool wide = false;
+  for (const BlockSpec& sp : specs)
+    wide |= tile_wide(sp.lda, complex ? 16 : 8) || tile_wide(sp.ldb, complex ? 16 : 8);
+  if (wide) persistent = false;
+  kernels_ = batched_kernels(complex, desc_.conjA != 0, opA == SPLA_OP_NONE ? MNMajor : KMajor,
+                             sched.cfg,
+                             wide ? BatchWide : persistent ? BatchPersistent : BatchGrouped);
   // GEMM workgroups: one per item (grouped) or one per slot (persistent)
   numItems_ = sched.items.empty() ? 0u
                                   : static_cast<unsigned>(persistent ? sched.slotStart.size() - 1
