@@ -67,7 +67,9 @@ __device__ __forceinline__ void map_block(const GemmDesc& d, int& s, int& tm, in
   const int G = gridDim.x;
   const int bid = blockIdx.x;
   int lin = bid;
-  if ((G & 7) == 0) lin = (bid & 7) * (G >> 3) + (bid >> 3);
+  // With a fill mode the active tiles of a contiguous share differ from XCD to XCD:
+  // there the dispatcher's round-robin order balances them.
+  if ((G & 7) == 0 && d.fillMode == FillFull) lin = (bid & 7) * (G >> 3) + (bid >> 3);
   const int tilesPerSplit = d.tilesM * d.tilesN;
   s = lin / tilesPerSplit;
   const int t = lin - s * tilesPerSplit;

@@ -392,7 +392,7 @@ void BatchPlan::execute() {
       if (mask[i]) splitSeconds += lower;
       (mask[i] ? split : fp64).push_back(b);
     }
-    allFp64 = split.empty() || splitSeconds >= 0.8 * best_schedule(split).modelSeconds;
+    allFp64 = split.empty() || splitSeconds >= 0.95 * best_schedule(split).modelSeconds;
   }
   if (allFp64) {
     // the grouped GEMM and the split reduction, replayed from the graph

@@ -115,7 +115,7 @@ private:
   std::size_t deviceMemory_ = 0;
 
   spla_amd::Tuner tuner_;
-  double batchEfficiency_[2] = {0.75, 0.55};  // TileL, TileM
+  double batchEfficiency_[2] = {0.93, 0.90};  // TileL, TileM
   bool batchPersistent_ = false;
   int gemmMode_ = 0;
   double splitTolerance_ = 1e-14;

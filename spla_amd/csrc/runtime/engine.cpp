@@ -186,7 +186,9 @@ void enqueue_device_product(SplaOperation opA, SplaOperation opB, int64_t m, int
 
   const int la = (opA == SPLA_OP_NONE) ? MNMajor : KMajor;
   const int lb = (opB == SPLA_OP_NONE) ? KMajor : MNMajor;
-  GemmPlan plan = ctx.tuner().plan(cplx, la, lb, m, n, k, ctx.num_cus(), wholeChip);
+  GemmPlan plan =
+      ctx.tuner().plan(cplx, la, lb, m, n, k, ctx.num_cus(), wholeChip, f32 ? 4 : 8,
+                       PlanFill{d.fillMode, d.fillRowOff, d.fillColOff});
   // Small m, n with a long reduction on a whole device: HBM-bound, streamed by
   // the skinny kernel (one workgroup per split, no LDS staging).
   // (kSkinnyMinKp / kSkinnyMinKpPerSplit >= 2: always several splits)

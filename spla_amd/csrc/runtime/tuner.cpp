@@ -42,13 +42,15 @@ int env_tile() {
   return -1;
 }
 
-}  // namespace
-
-GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, int forceCfg,
-                   int forceSplits, const double* effByCfg, bool wholeChip) {
+// Plan and time of a coarse model that the forced plans, the block products of a
+// batch and the automatic mode's choice of arithmetic are made with: waves of
+// workgroups over the resident slots, no fill mode.
+GemmPlan plan_coarse(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, int forceCfg,
+                     int forceSplits, bool wholeChip) {
   const int64_t Mp = complex ? 2 * m : m;
   const int64_t Kp = complex ? 2 * k : k;
-  const int cands[] = {TileL, TileM, TileXL};
+  constexpr int cands[] = {TileL, TileM, TileXL};
+  constexpr double rate[] = {0.8, 0.55, 0.85};  // L, M, XL
   GemmPlan best;
   best.estSeconds = 1e300;
   for (int cfg : cands) {
@@ -61,7 +63,7 @@ GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, in
     const int64_t kBlocks = std::max<int64_t>(1, (Kp + ts.bk - 1) / ts.bk);
     const int bpc = blocks_per_cu(cfg);
     const int64_t slots = static_cast<int64_t>(numCUs) * bpc;
-    const double eff = effByCfg ? effByCfg[cfg] : 0.8;
+    const double eff = rate[cfg];
     // split factors: every split keeps at least 8 k-blocks; up to 64, or, for a
     // product that has the device to itself, as many as fill the resident workgroup
     // slots when there are few tiles (small m, n and a long reduction: HBM-bound,
@@ -119,22 +121,118 @@ GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, in
   return best;
 }
 
-double Tuner::efficiency(int cfg) {
-  switch (cfg) {
-    case TileXL:
-      return 0.85;
-    case TileM:
-      return 0.55;
-    default:
-      return 0.8;
+// Bytes of partial sums. The allocation-free entry point (complex doubles) holds
+// 64 MiB: a product whose coarse plan fits keeps within it.
+constexpr double kSmallWorkspace = 64.0 * (1 << 20);
+constexpr double kLargestWorkspace = 256.0 * (1 << 20);
+
+}  // namespace
+
+int64_t plan_active_tiles(int64_t m, int64_t n, int rows, int cols, const PlanFill& fill) {
+  const int64_t tilesM = (m + rows - 1) / rows, tilesN = (n + cols - 1) / cols;
+  if (fill.mode == FillFull) return tilesM * tilesN;
+  int64_t count = 0;
+  for (int64_t tn = 0; tn < tilesN; ++tn) {
+    const int64_t c = tn * cols + fill.colOff - fill.rowOff;
+    const int64_t nc = std::min<int64_t>(cols, n - tn * cols);
+    if (fill.mode == FillUpper)  // first row of the tile before the last column's diagonal entry
+      count += std::max<int64_t>(0, std::min(tilesM, (c + nc + rows - 1) / rows));
+    else if (c < m)  // last row of the tile past the first column's diagonal entry
+      count += tilesM - std::max<int64_t>(0, c) / rows;
   }
+  return count;
 }
 
+// Whole-device plans. Every workgroup of a launch computes one tile over one
+// split. With one round of resident workgroups a CU has q of them side by side;
+// a single one keeps its matrix cores busy to 0.88 (M) or 0.85 (L) of what a full
+// CU reaches (700 x 700 x 30011 complex on M tiles: 242 workgroups 1.82 ms, 726
+// 1.72 ms). Past that the dispatcher hands workgroups out as slots free up, and a
+// last, partial round can land more than once on the same CU (1210 workgroups:
+// 2.07 ms), which many short rounds avoid (5808: 1.68 ms). Splitting the
+// reduction costs the write and read of the partial sums and a launch.
+GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, int forceCfg,
+                   int forceSplits, const double* effByCfg, bool wholeChip, int scalarBytes,
+                   const PlanFill& fill) {
+  const GemmPlan coarse =
+      plan_coarse(complex, m, n, k, numCUs, forceCfg, forceSplits, wholeChip);
+  if (!wholeChip || forceCfg >= 0 || forceSplits > 0) return coarse;
+  constexpr double kWorkgroupSeconds = 2.5e-6;  // address set-up, first loads, epilogue
+  constexpr double kBlockSeconds = 0.6e-6;  // shortest k-block of one workgroup (latency)
+  constexpr double kReduceLaunchSeconds = 4.0e-6;
+  const int64_t Mp = complex ? 2 * m : m;
+  const int64_t Kp = complex ? 2 * k : k;
+  const double sums = static_cast<double>(Mp) * n * scalarBytes;  // bytes of one split
+  const bool small = complex && scalarBytes == 8 && coarse.splits * sums <= kSmallWorkspace;
+  const double limit = small ? kSmallWorkspace : kLargestWorkspace;
+  const double bytes = static_cast<double>(m + n) * k * scalarBytes * (complex ? 2 : 1);
+  GemmPlan best = coarse;
+  double bestSeconds = 1e300, fullSeconds = 1e300;
+  for (int cfg : {TileL, TileM}) {
+    const TileShape ts = tile_shape(cfg);
+    const int rows = complex ? ts.bm / 2 : ts.bm;
+    const int64_t bk = ts.bk * (scalarBytes == 4 ? 2 : 1);  // a k-block is 128 bytes of a row
+    const int64_t tilesM = (m + rows - 1) / rows, tilesN = (n + ts.bn - 1) / ts.bn;
+    const int64_t allTiles = tilesM * tilesN;
+    const int64_t tiles = std::max<int64_t>(1, plan_active_tiles(m, n, rows, ts.bn, fill));
+    const int64_t kBlocks = std::max<int64_t>(1, (Kp + bk - 1) / bk);
+    const int perCU = blocks_per_cu(cfg);
+    const int64_t slots = static_cast<int64_t>(numCUs) * perCU;
+    const double peak = kPeakPerCU * (8.0 / scalarBytes) * effByCfg[cfg];
+    const double lone = cfg == TileL ? 0.85 : 0.88;
+    const int64_t maxSplits = std::max<int64_t>(
+        1, std::min<int64_t>(kBlocks / 8, std::max<int64_t>(64, 4 * slots / tiles)));
+    int64_t lastSplits = 0;
+    for (int64_t s = 1; s <= maxSplits; s += std::max<int64_t>(1, s / 32)) {
+      const int64_t kb = (kBlocks + s - 1) / s;
+      const int64_t splits = (kBlocks + kb - 1) / kb;  // no empty split
+      if (splits == lastSplits || allTiles * splits > (int64_t(1) << 31) - 1) continue;
+      lastSplits = splits;
+      if (splits > 1 && splits * sums > limit) break;
+      const double work = 2.0 * ts.bm * ts.bn * bk * kb / peak;  // one workgroup on a full CU
+      auto seconds = [&](int64_t groups) {
+        const int64_t rounds = groups / slots, rest = groups % slots;
+        double t = rounds * perCU * work + (rounds > 0 ? (0.7 + 0.3 * rounds) : 0.0) *
+                                               kWorkgroupSeconds;
+        if (rest > 0) {
+          const int64_t spread = (rest + numCUs - 1) / numCUs;
+          const int64_t q = rounds > 0 ? std::min<int64_t>(perCU, spread + 1) : spread;
+          t += std::max(q * work / (q == 1 ? lone : 1.0), kb * kBlockSeconds) + kWorkgroupSeconds;
+        }
+        const double inFlight = std::min(1.0, groups / (2.0 * numCUs));
+        t = std::max(t, bytes / (kHbmBytesPerSecond * inFlight)) + kLaunchSeconds;
+        if (splits > 1)
+          t += (1.5 * splits + 2) * sums / kHbmBytesPerSecond + kReduceLaunchSeconds;
+        return t;
+      };
+      const double t = seconds(tiles * splits);
+      fullSeconds = std::min(fullSeconds, seconds(allTiles * splits));
+      if (t < bestSeconds * 0.999) {
+        bestSeconds = t;
+        best.cfg = cfg;
+        best.splits = static_cast<int>(splits);
+        best.kSplit = kb * bk;
+        best.tilesM = static_cast<int>(tilesM);
+        best.tilesN = static_cast<int>(tilesN);
+      }
+    }
+  }
+  // what the automatic mode compares the split form with: its margin (0.8) was
+  // drawn for the coarse model's rates, 0.84 of those reached now
+  best.estSeconds = std::min(coarse.estSeconds, fullSeconds / 0.84);
+  return best;
+}
+
+// Measured on long reductions: 2048 x 2048 x 2e4, complex and real, 74.2-75.6
+// TFLOP/s on L tiles and 71.7-72.4 on M tiles.
+double Tuner::efficiency(int cfg) { return cfg == TileM ? 0.91 : 0.95; }
+
 GemmPlan Tuner::plan(bool complex, int layoutA, int layoutB, int64_t m, int64_t n, int64_t k,
-                     int numCUs, bool wholeChip) {
+                     int numCUs, bool wholeChip, int scalarBytes, const PlanFill& fill) {
   const int forceCfg = env_tile();
   const int forceSplits = env_int("SPLA_AMD_SPLITS", 0);
-  const Key key{complex, layoutA, layoutB, m, n, k, numCUs, wholeChip};
+  const Key key{complex, layoutA, layoutB, m, n, k, numCUs, wholeChip, scalarBytes, fill.mode,
+                fill.mode == FillFull ? 0 : fill.colOff - fill.rowOff};
   std::lock_guard<std::mutex> guard(lock_);
   if (forceCfg < 0 && forceSplits <= 0) {
     auto it = cache_.find(key);
@@ -142,7 +240,8 @@ GemmPlan Tuner::plan(bool complex, int layoutA, int layoutB, int64_t m, int64_t 
   }
   double eff[NumTileConfigs];
   for (int c = 0; c < NumTileConfigs; ++c) eff[c] = efficiency(c);
-  GemmPlan p = plan_gemm(complex, m, n, k, numCUs, forceCfg, forceSplits, eff, wholeChip);
+  GemmPlan p = plan_gemm(complex, m, n, k, numCUs, forceCfg, forceSplits, eff, wholeChip, scalarBytes,
+                         fill);
   if (forceCfg < 0 && forceSplits <= 0) cache_[key] = p;
   return p;
 }

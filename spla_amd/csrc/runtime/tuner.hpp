@@ -1,8 +1,8 @@
 // Tile-shape and split-K planner of the FP64 MFMA GEMM.
 //
 // A plan is picked by a cost model of the launch: for every tile shape and
-// split factor the model counts waves of workgroups over the CUs, the time of
-// one wave at the shape's sustained MFMA rate, tile padding waste, and the
+// split factor the model counts the workgroups of the active tiles over the CUs,
+// their time at the shape's sustained MFMA rate, tile padding waste, and the
 // HBM time of the split-K reduction; the cheapest plan wins. Plans are cached
 // per problem key and depend only on the shape, so that repeated calls of one
 // product split the reduction alike and return bitwise identical results (the
@@ -26,25 +26,39 @@ struct GemmPlan {
   double estSeconds = 0.0;
 };
 
+// Part of C that a product needs (the kernels' TileFill and offsets).
+struct PlanFill {
+  int mode = 0;
+  int64_t rowOff = 0, colOff = 0;
+};
+
 class Tuner {
 public:
   // complex: complex operands; m, n, k in elements; numCUs of the device.
   // wholeChip: the product has the device to itself (a single call); false for the
   // block products of a batch, which run side by side on several streams.
+  // scalarBytes: 8 or 4 (single precision). fill: whole-device plans count the tiles
+  // it leaves.
   GemmPlan plan(bool complex, int layoutA, int layoutB, int64_t m, int64_t n, int64_t k,
-                int numCUs, bool wholeChip = true);
+                int numCUs, bool wholeChip = true, int scalarBytes = 8,
+                const PlanFill& fill = PlanFill());
 
   // Sustained fraction of the per-CU FP64 matrix rate assumed for a tile config.
   static double efficiency(int cfg);
 
 private:
-  using Key = std::tuple<bool, int, int, int64_t, int64_t, int64_t, int, bool>;
+  using Key = std::tuple<bool, int, int, int64_t, int64_t, int64_t, int, bool, int, int, int64_t>;
   std::mutex lock_;
   std::map<Key, GemmPlan> cache_;
 };
 
+// Tiles of rows x cols elements that the fill mode leaves active (the kernels'
+// tile_active over all tiles of an m x n matrix).
+int64_t plan_active_tiles(int64_t m, int64_t n, int rows, int cols, const PlanFill& fill);
+
 // Pure cost model (no state), exposed for tests.
 GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, int forceCfg,
-                   int forceSplits, const double* effByCfg, bool wholeChip = true);
+                   int forceSplits, const double* effByCfg, bool wholeChip = true,
+                   int scalarBytes = 8, const PlanFill& fill = PlanFill());
 
 }  // namespace spla_amd
