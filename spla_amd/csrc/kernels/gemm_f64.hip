@@ -188,19 +188,20 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(GemmDesc d, int tile
   store_result<S, CPLX>(d, i, j, re, im);
 }
 
-// Many splits over few elements (small m, n, long reduction): 16 elements per
-// block, 16 split groups per element. Group g sums splits g, g + 16, g + 32, ...
-// in order and the 16 group sums are added in group order, so the result is
-// bitwise reproducible; every split is read by 16 consecutive elements at once.
-constexpr int kWideElems = 16;
-constexpr int kWideGroups = 16;
-template <typename S, bool CPLX>
+// Many splits over few elements (small m, n, long reduction): ELEMS elements per
+// block, 256 / ELEMS split groups per element. Group g sums splits g, g + groups,
+// ... in order and the group sums are added pairwise, so the result is bitwise
+// reproducible. Bound by latency: with 16 elements per block the 256 sums of a 16 x
+// 16 product over 1024 splits ran in 16 blocks of 64 loads after each other (30
+// us); four take 64 blocks of 8 loads over its 512 splits now (4.4 us).
+template <typename S, bool CPLX, int ELEMS>
 __global__ void __launch_bounds__(256) splitk_reduce_wide_kernel(GemmDesc d, int tileRows,
                                                                  int tileCols) {
-  __shared__ S part[kWideGroups][kWideElems][2];
-  const int e = threadIdx.x % kWideElems;
-  const int g = threadIdx.x / kWideElems;
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * kWideElems + e;
+  constexpr int kGroups = 256 / ELEMS;
+  __shared__ S part[kGroups][ELEMS][2];
+  const int e = threadIdx.x % ELEMS;
+  const int g = threadIdx.x / ELEMS;
+  const int64_t idx = static_cast<int64_t>(blockIdx.x) * ELEMS + e;
   const int64_t total = static_cast<int64_t>(d.m) * d.n;
   bool live = idx < total;
   const int i = live ? static_cast<int>(idx % d.m) : 0;
@@ -216,23 +217,22 @@ __global__ void __launch_bounds__(256) splitk_reduce_wide_kernel(GemmDesc d, int
   if (live) {
     const int64_t stride = static_cast<int64_t>(d.n) * d.Mp;
     const S* w = static_cast<const S*>(d.work) + static_cast<int64_t>(j) * d.Mp + (CPLX ? 2 * i : i);
-    for (int sp = g; sp < d.splits; sp += kWideGroups) {
+#pragma unroll 8
+    for (int sp = g; sp < d.splits; sp += kGroups) {
       re += w[sp * stride];
       if (CPLX) im += w[sp * stride + 1];
     }
   }
   part[g][e][0] = re;
   part[g][e][1] = im;
-  __syncthreads();
-  if (g == 0 && live) {
-    S sr = part[0][e][0], si = part[0][e][1];
-#pragma unroll
-    for (int q = 1; q < kWideGroups; ++q) {
-      sr += part[q][e][0];
-      si += part[q][e][1];
+  for (int half = kGroups / 2; half > 0; half /= 2) {
+    __syncthreads();
+    if (g < half) {
+      part[g][e][0] += part[g + half][e][0];
+      if (CPLX) part[g][e][1] += part[g + half][e][1];
     }
-    store_result<S, CPLX>(d, i, j, sr, si);
   }
+  if (g == 0 && live) store_result<S, CPLX>(d, i, j, part[0][e][0], part[0][e][1]);
 }
 
 // C <- beta * C (k == 0 or alpha == 0); beta == 0 writes zeros without reading C.
@@ -356,14 +356,17 @@ hipError_t launch_splitk_reduce_s(const GemmDesc& d, bool complex, int cfg, hipS
   const TileShape ts = tile_shape(cfg);
   const int tileRows = complex ? ts.bm / 2 : ts.bm;
   const int64_t total = static_cast<int64_t>(d.m) * d.n;
-  if (d.splits > 64) {  // only the whole-device plans of small m, n split this far
-    const dim3 wide(static_cast<unsigned>((total + kWideElems - 1) / kWideElems));
-    if (complex)
-      hipLaunchKernelGGL((splitk_reduce_wide_kernel<S, true>), wide, dim3(256), 0, stream, d,
-                         tileRows, ts.bn);
-    else
-      hipLaunchKernelGGL((splitk_reduce_wide_kernel<S, false>), wide, dim3(256), 0, stream, d,
-                         tileRows, ts.bn);
+  // One element per thread fills the chip from 16384 elements on; below, up to
+  // 16 splits after each other still cost less than the group sums.
+  if (d.splits > 64 || (d.splits > 16 && total < 16384)) {
+    const bool few = total <= 4096;
+    const int elems = few ? 4 : 16;
+    const dim3 wide(static_cast<unsigned>((total + elems - 1) / elems));
+    auto* kernel = complex ? (few ? splitk_reduce_wide_kernel<S, true, 4>
+                                  : splitk_reduce_wide_kernel<S, true, 16>)
+                           : (few ? splitk_reduce_wide_kernel<S, false, 4>
+                                  : splitk_reduce_wide_kernel<S, false, 16>);
+    hipLaunchKernelGGL(kernel, wide, dim3(256), 0, stream, d, tileRows, ts.bn);
     return hipGetLastError();
   }
   const dim3 grid(static_cast<unsigned>((total + 255) / 256));

@@ -5,23 +5,32 @@
 // flop per byte, below the FP64 matrix ridge (78.6 TFLOP/s / 8 TB/s = 9.8) for
 // m = n <= 39.
 //
-// Each wave owns the whole (embedded) m x n output in FM x FN MFMA fragments
-// and streams a share of the reduction straight from global memory into the
-// MFMA operand registers: no LDS staging and no barrier per k-block. A wave
-// step covers 16 embedded reduction indices, i.e. one 128-byte line of every
-// row of A and B it reads; DEPTH steps of loads are in flight per wave
-// (register ring), so that the CU keeps ~100-200 KB of loads outstanding.
-// The four waves of a workgroup interleave their steps over the workgroup's
-// reduction range and add their accumulators through LDS in wave order at the
-// end; the workgroup's sum is one split-K partial, which the fixed-order
-// reduction kernel adds to the others with alpha / beta.
+// Each wave owns the whole m x n output in FM x FN MFMA fragments of 16 x 16
+// elements. It streams chunks of 128 bytes of every row, eight rows per load
+// instruction, through registers and a part of LDS of its own into the layout of
+// the MFMA operands: no barrier in the loop, the loads of the next chunk in flight
+// during the MFMAs of this one. The waves of all workgroups take the chunks in
+// turn, so that the chip reads one moving window of every row.
 //
-// Fragment layout (v_mfma_f64_16x16x4_f64): lane l holds A[l % 16][l / 16] and
-// B[l / 16][l % 16]; the accumulator holds rows l / 16 + 4 r of column l % 16.
-// Complex products use the real embedding of the tiled kernels: fragment rows
-// 0-7 are the real and 8-15 the imaginary parts of 8 complex rows; a lane reads
-// the (re, im) pair of one element and the imaginary rows swap it and flip
-// signs lane-constantly (conjugation of A and / or B).
+// Why through LDS: a fragment read straight into registers takes 64 bytes of 16
+// rows per load instruction, half a cache line. Measured (one card, kernel alone,
+// same accumulation): complex m = n = 16, k = 8e6 745 -> 580 us (5.5 -> 7.1 TB/s),
+// m = n = 32, k = 4e6 1037 -> 606 us (3.9 -> 6.8 TB/s); 256-byte chunks, two
+// chunks in flight and four workgroups per CU instead of two are 1 to 5 % slower,
+// loads without the non-temporal hint 10 to 13 %.
+//
+// Small outputs (GROUPS > 1): m, n <= 16 / GROUPS. A fragment holds GROUPS
+// stretches of 128 bytes of its 16 / GROUPS rows; the products of equal stretches
+// lie in the diagonal blocks of the accumulator and are added at the end. With one
+// stretch the matrix cores would spend 16 x 16 outputs on m x n and bound the
+// product (m = n = 1: 1.2 TB/s).
+//
+// Arithmetic as in tile_mma.hpp: complex operands are not expanded (four MFMAs per
+// pair of fragments, the MFMA's own negation), B is the first MFMA operand, lane
+// (kk, l16) holds rows kk + 4 r of D (columns of C) and column l16 (row of C).
+// Two accumulators per output (complex: the two products of each component, real:
+// the two elements of a chunk's 16-byte pieces) halve the length of the sums, where
+// there are registers for them.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -36,220 +45,252 @@ namespace {
 using namespace tile;
 
 constexpr int kWaves = 4;
-constexpr int kStep = 16;  // embedded reduction indices per wave step
+constexpr int kChunkRowBytes = 128;  // of one row and stretch
 
-// Two waves per SIMD (at most 256 registers per lane): with one, the m = n = 32
-// complex product streamed 8 % less (3.57 vs 3.92 TB/s), its MFMAs and loads
-// waiting on each other in the single wave.
-template <bool CPLX, int FM, int FN, int DEPTH>
+// LINES: 128-byte stretches of a row that follow each other in a chunk; ALIGNED: every
+// row starts on a cache line (see rows_aligned).
+template <bool CPLX, bool CONJ, int FM, int FN, int GROUPS, int LINES, bool ALIGNED>
 __global__ void __launch_bounds__(kWaves * 64, 2) skinny_gemm_kernel(GemmDesc d) {
-  constexpr int ROWS = CPLX ? 8 : 16;  // rows of A per fragment (complex: re / im pairs)
+  static_assert(GROUPS == 1 || (FM == 1 && FN == 1), "stretches share one fragment");
+  static_assert(GROUPS == 1 || LINES == 1, "one or the other");
+  constexpr int kComps = CPLX ? 2 : 1;
+  constexpr int kElem = 8 * kComps;
+  constexpr int kRows = 16 / GROUPS;  // rows of A or columns of B in a fragment
+  constexpr int kChunk = kChunkRowBytes * GROUPS * LINES;  // bytes of a row in one chunk
+  constexpr int kChunkElems = kChunk / kElem;
+  constexpr int kPerRow = kChunk / 16;      // 16-byte pieces of a row
+  constexpr int kLoadsA = 2 * FM * LINES, kLoads = 2 * (FM + FN) * LINES;  // per lane and chunk
+  constexpr int kLineBytes = 16 * (FM + FN) * kRowBytes;
+  constexpr int kStageBytes = LINES * kLineBytes;
+  constexpr int kSumBytes = FM * FN * kComps * 16 * 17 * 8;
+  constexpr int kWaveBytes = kStageBytes > kSumBytes ? kStageBytes : kSumBytes;
+  constexpr int kSums = 16 * FM * FN * kComps + 6 * kLoads < 200 ? 2 : 1;  // per output
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kWaves][kWaveBytes];
+  typedef double loose2 __attribute__((ext_vector_type(2), aligned(8)));
+
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15;
   const int kk = lane >> 4;
-  const bool imagRow = CPLX && l16 >= 8;
-  const int arow = CPLX ? (l16 & 7) : l16;
-  uint32_t sgn0 = 0, sgn1 = 0;
-  if (CPLX) {
-    if (!imagRow) {
-      sgn1 = (d.conjA == d.conjB) ? 0x80000000u : 0u;
-    } else {
-      sgn0 = d.conjA ? 0x80000000u : 0u;
-      sgn1 = d.conjB ? 0x80000000u : 0u;
-    }
-  }
-  const double* __restrict__ A = static_cast<const double*>(d.A);
-  const double* __restrict__ B = static_cast<const double*>(d.B);
-  const int64_t comps = CPLX ? 2 : 1;
-  const int64_t kBegin = static_cast<int64_t>(blockIdx.x) * d.kSplit;
-  const int64_t kEnd = min(d.Kp, kBegin + d.kSplit);
-  const int64_t steps = (kEnd - kBegin + kStep - 1) / kStep;
-  // this wave's steps: wave, wave + 4, wave + 8, ...
-  const int64_t mySteps = steps > wave ? (steps - wave + kWaves - 1) / kWaves : 0;
+  // chunks of this wave: id, id + waves, id + 2 waves, ...; the partial chunk at
+  // the end of the reduction goes to the wave whose turn it is
+  const int64_t chunks = d.k / kChunkElems;
+  const int64_t waves = static_cast<int64_t>(gridDim.x) * kWaves;
+  const int64_t id = static_cast<int64_t>(blockIdx.x) * kWaves + wave;
+  const int64_t mine = chunks > id ? (chunks - id + waves - 1) / waves : 0;
+  const bool tail = d.k % kChunkElems != 0 && chunks % waves == id;
 
-  // row / column bases of this lane; rows past m and columns past n read row /
-  // column 0 and are zeroed after the load, so that every load is issued
-  // unconditionally and the waits for the register ring stay static
-  const double* pa[FM];
-  bool va[FM];
-#pragma unroll
-  for (int f = 0; f < FM; ++f) {
-    const int r = ROWS * f + arow;
-    va[f] = r < d.m;
-    pa[f] = A + static_cast<int64_t>(va[f] ? r : 0) * d.lda * comps;
-  }
-  const double* pb[FN];
-  bool vb[FN];
-#pragma unroll
-  for (int g = 0; g < FN; ++g) {
-    const int c = 16 * g + l16;
-    vb[g] = c < d.n;
-    pb[g] = B + static_cast<int64_t>(vb[g] ? c : 0) * d.ldb * comps;
-  }
-
-  typedef double dbl2v __attribute__((ext_vector_type(2)));
-  dbl2v ra[DEPTH][FM][2], rb[DEPTH][FN][2];
-  dbl4 acc[FM][FN];
-#pragma unroll
-  for (int f = 0; f < FM; ++f)
-#pragma unroll
-    for (int g = 0; g < FN; ++g) acc[f][g] = dbl4{0.0, 0.0, 0.0, 0.0};
-
-  // loads of wave step t into a ring slot; sub-block h of the step holds
-  // embedded indices q0 + 8 h + 2 kk and q0 + 8 h + 2 kk + 1. Indices past kEnd
-  // (the range's tail, and the steps past the wave's last one that the ring's
-  // tail loads) read the range's first element, rows past m and columns past n
-  // read row / column 0; compute() zeroes all of them where it uses the values
-  // (zeroing right after the load would make the wave wait for each load), so
-  // the ring runs without a branch and the surplus steps add zeros.
-  auto step_q = [&](int64_t t, int h) {
-    return kBegin + (wave + t * kWaves) * static_cast<int64_t>(kStep) + 8 * h + 2 * kk;
+  // Piece u of a lane: row and 16-byte piece of A or B, and where it lies in LDS.
+  // Rows past the operand's last one read that one: they feed outputs that are
+  // not stored.
+  constexpr int kLoadRows = GROUPS == 1 ? 64 / kPerRow : 1;  // of one load instruction
+  auto piece_row = [&](int u) {
+    const int v = u < kLoadsA ? u : u - kLoadsA;
+    return GROUPS == 1 ? v * kLoadRows + lane / kPerRow : (v * 64 + lane) / kPerRow;
   };
-  auto load = [&](int64_t t, auto& sa, auto& sb) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t q = step_q(t, h);
-      const bool in0 = q < kEnd, in1 = q + 1 < kEnd;  // complex: in1 == in0 (q, kEnd even)
-      const int64_t qc = in0 ? q : kBegin;            // a valid address for every lane
-      const int64_t qc1 = in1 ? q + 1 : qc;
-#pragma unroll
-      for (int f = 0; f < FM; ++f) {
-        if (CPLX) {
-          sa[f][h] = *reinterpret_cast<const dbl2v*>(pa[f] + qc);
-        } else {
-          sa[f][h].x = pa[f][qc];
-          sa[f][h].y = pa[f][qc1];
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < FN; ++g) {
-        if (CPLX) {
-          sb[g][h] = *reinterpret_cast<const dbl2v*>(pb[g] + qc);
-        } else {
-          sb[g][h].x = pb[g][qc];
-          sb[g][h].y = pb[g][qc1];
-        }
-      }
-    }
+  auto piece_col = [&](int u) {
+    const int v = u < kLoadsA ? u : u - kLoadsA;
+    return GROUPS == 1 ? lane % kPerRow : (v * 64 + lane) % kPerRow;
   };
-  auto compute = [&](int64_t t, const auto& sa, const auto& sb) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t q = step_q(t, h);
-      const bool in0 = q < kEnd, in1 = q + 1 < kEnd;
-      double a0[FM], a1[FM], b0[FN], b1[FN];
-#pragma unroll
-      for (int f = 0; f < FM; ++f) {
-        const dbl2v v = sa[f][h];
-        const double vx = (va[f] && in0) ? v.x : 0.0;
-        const double vy = (va[f] && in1) ? v.y : 0.0;
-        if (CPLX) {
-          const double x = imagRow ? vy : vx;
-          const double y = imagRow ? vx : vy;
-          a0[f] = flip_sign(x, sgn0);
-          a1[f] = flip_sign(y, sgn1);
-        } else {
-          a0[f] = vx;
-          a1[f] = vy;
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < FN; ++g) {
-        b0[g] = (vb[g] && in0) ? sb[g][h].x : 0.0;
-        b1[g] = (vb[g] && in1) ? sb[g][h].y : 0.0;
-      }
-#pragma unroll
-      for (int f = 0; f < FM; ++f)
-#pragma unroll
-        for (int g = 0; g < FN; ++g) acc[f][g] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[f], b0[g], acc[f][g], 0, 0, 0);
-#pragma unroll
-      for (int f = 0; f < FM; ++f)
-#pragma unroll
-        for (int g = 0; g < FN; ++g) acc[f][g] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[f], b1[g], acc[f][g], 0, 0, 0);
-    }
+  auto slot = [&](int u) {
+    const int row = piece_row(u), col = piece_col(u), first = u < kLoadsA ? 0 : 16 * FM;
+    return (GROUPS == 1 ? col / 8 * kLineBytes + (first + row) * kRowBytes
+                        : (first + col / 8 * kRows + row) * kRowBytes) +
+           16 * (col % 8);
   };
-
-  if (mySteps > 0) {
+  const char* p[kLoads];
 #pragma unroll
-    for (int u = 0; u < DEPTH; ++u) load(u, ra[u], rb[u]);
-    for (int64_t base = 0; base < mySteps; base += DEPTH) {
-#pragma unroll
-      for (int u = 0; u < DEPTH; ++u) {
-        compute(base + u, ra[u], rb[u]);
-        load(base + u + DEPTH, ra[u], rb[u]);
-      }
-    }
+  for (int u = 0; u < kLoads; ++u) {
+    const int row = piece_row(u);
+    p[u] = u < kLoadsA ? static_cast<const char*>(d.A) + min(row, d.m - 1) * d.lda * kElem
+                       : static_cast<const char*>(d.B) + min(row, d.n - 1) * d.ldb * kElem;
+    p[u] += 16 * piece_col(u);
   }
+  unsigned char* const own = lds[wave];
+  const unsigned char* const operand = own + l16 * kRowBytes + 16 * kk;
 
-  // the four waves' sums, added in wave order
-  __shared__ dbl4 part[kWaves - 1][FM][FN][64];
-  if (wave > 0) {
+  dbl4 re[kSums][FM][FN], im[kSums][CPLX ? FM : 1][CPLX ? FN : 1];
+#pragma unroll
+  for (int h = 0; h < kSums; ++h)
 #pragma unroll
     for (int f = 0; f < FM; ++f)
 #pragma unroll
-      for (int g = 0; g < FN; ++g) part[wave - 1][f][g][lane] = acc[f][g];
+      for (int g = 0; g < FN; ++g) {
+        re[h][f][g] = dbl4{0.0, 0.0, 0.0, 0.0};
+        if constexpr (CPLX) im[h][f][g] = dbl4{0.0, 0.0, 0.0, 0.0};
+      }
+  // one chunk, from its registers through LDS; `next` runs once the registers are free
+  auto compute = [&](const dbl2 (&x)[kLoads], auto next) {
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) *reinterpret_cast<dbl2*>(own + slot(u)) = x[u];
+    __builtin_amdgcn_sched_barrier(0);
+    next();
+    // LDS serves a wave's own accesses in order: only the compiler must keep it
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int s = 0; s < 2 * LINES; ++s) {
+      const unsigned char* const from = operand + s / 2 * kLineBytes + 64 * (s % 2);
+      dbl2 a[FM], b[FN];
+#pragma unroll
+      for (int f = 0; f < FM; ++f)
+        a[f] = *reinterpret_cast<const dbl2*>(from + f * 16 * kRowBytes);
+#pragma unroll
+      for (int g = 0; g < FN; ++g)
+        b[g] = *reinterpret_cast<const dbl2*>(from + (FM + g) * 16 * kRowBytes);
+#pragma unroll
+      for (int q = 0; q < 2 * kComps; ++q)
+#pragma unroll
+        for (int f = 0; f < FM; ++f)
+#pragma unroll
+          for (int g = 0; g < FN; ++g) {
+            constexpr int h = kSums - 1;  // the second sum
+            if constexpr (!CPLX) {
+              re[q * h][f][g] = mfma16x16x4<false>(b[g][q], a[f][q], re[q * h][f][g]);
+            } else {
+              if (q == 0) re[0][f][g] = mfma16x16x4<false>(b[g][0], a[f][0], re[0][f][g]);
+              if (q == 1) im[0][f][g] = mfma16x16x4<CONJ>(b[g][0], a[f][1], im[0][f][g]);
+              if (q == 2) re[h][f][g] = mfma16x16x4<!CONJ>(b[g][1], a[f][1], re[h][f][g]);
+              if (q == 3) im[h][f][g] = mfma16x16x4<false>(b[g][1], a[f][0], im[h][f][g]);
+            }
+          }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) p[u] += id * kChunk;
+  if (mine > 0) {
+    dbl2 x[kLoads];
+    auto load = [&]() {
+#pragma unroll
+      for (int u = 0; u < kLoads; ++u) {
+        const loose2* q = reinterpret_cast<const loose2*>(p[u]);
+        x[u] = ALIGNED ? __builtin_nontemporal_load(q) : *q;
+      }
+    };
+    load();
+    const int64_t step = waves * kChunk;
+    for (int64_t c = 1; c < mine; ++c) {
+#pragma unroll
+      for (int u = 0; u < kLoads; ++u) p[u] += step;
+      compute(x, load);
+    }
+    compute(x, [] {});
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) p[u] += step;
   }
+  if (tail) {  // p is at the partial chunk: elements past the reduction are zero
+    const int left = static_cast<int>(d.k % kChunkElems) * kComps;  // doubles
+    dbl2 x[kLoads];
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      const int at = 2 * piece_col(u);
+      const double* q = reinterpret_cast<const double*>(p[u]);
+      x[u] = dbl2{0.0, 0.0};
+      if (at < left) x[u][0] = q[0];
+      if (at + 1 < left) x[u][1] = q[1];
+    }
+    compute(x, [] {});
+  }
+
+  // The sums of the four waves and of the stretches, in this order, through LDS.
   __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int w = 0; w < kWaves - 1; ++w)
-#pragma unroll
-    for (int f = 0; f < FM; ++f)
-#pragma unroll
-      for (int g = 0; g < FN; ++g) acc[f][g] += part[w][f][g][lane];
-
-  // accumulator rows kk + 4 r of column l16 (see tile_mma.hpp for_each)
-  double* work = static_cast<double*>(d.work) + static_cast<int64_t>(blockIdx.x) * d.n * d.Mp;
+  double* sums = reinterpret_cast<double*>(own);
 #pragma unroll
   for (int f = 0; f < FM; ++f)
 #pragma unroll
-    for (int g = 0; g < FN; ++g) {
-      const int j = 16 * g + l16;
-      if (j >= d.n) continue;
-      const dbl4 v = acc[f][g];
-      if (CPLX) {
-        const int base = 8 * f;
-        if (base + kk < d.m) store_work<double, true>(work, d.Mp, base + kk, j, v[0], v[2]);
-        if (base + kk + 4 < d.m) store_work<double, true>(work, d.Mp, base + kk + 4, j, v[1], v[3]);
-      } else {
+    for (int g = 0; g < FN; ++g)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (16 * f + kk + 4 * r < d.m)
-            store_work<double, false>(work, d.Mp, 16 * f + kk + 4 * r, j, v[r], 0.0);
+      for (int r = 0; r < 4; ++r) {
+        double* s = sums + ((f * FN + g) * kComps * 16 + kk + 4 * r) * 17 + l16;
+        s[0] = kSums == 2 ? re[0][f][g][r] + re[kSums - 1][f][g][r] : re[0][f][g][r];
+        if constexpr (CPLX)
+          s[16 * 17] = kSums == 2 ? im[0][f][g][r] + im[kSums - 1][f][g][r] : im[0][f][g][r];
       }
-    }
+  __syncthreads();
+  const bool flip = CPLX && (CONJ ? !d.conjA : (d.conjA && d.conjB));  // see TileMma::flip_result
+  double* work = static_cast<double*>(d.work) + static_cast<int64_t>(blockIdx.x) * d.n * d.Mp;
+  for (int e = threadIdx.x; e < d.n * d.Mp; e += kWaves * 64) {
+    const int j = e / d.Mp;
+    const int i = (e % d.Mp) / kComps, c = (e % d.Mp) % kComps;
+    const int at = ((i / 16 * FN + j / 16) * kComps + c) * 16 * 17 + (j % 16) * 17 + i % 16;
+    double sum = 0.0;
+    for (int w = 0; w < kWaves; ++w)
+#pragma unroll
+      for (int s = 0; s < GROUPS; ++s)
+        sum += reinterpret_cast<const double*>(lds[w])[at + s * kRows * 18];
+    work[e] = flip && c ? -sum : sum;
+  }
 }
 
-template <bool CPLX, int FM, int FN>
-hipError_t launch_fm_fn(const GemmDesc& d, hipStream_t stream) {
-  // loads in flight per wave: DEPTH steps of (FM + FN) x 2 x 16 bytes per lane
-  // (the largest ring that fits two waves per SIMD; measured 2 over 3 for FM + FN > 4)
-  constexpr int DEPTH = (FM + FN) <= 3 ? 6 : ((FM + FN) <= 4 ? 4 : 2);
-  hipLaunchKernelGGL((skinny_gemm_kernel<CPLX, FM, FN, DEPTH>), dim3(d.splits),
-                     dim3(kWaves * 64), 0, stream, d);
+// Rows that do not start on cache lines: every 128-byte stretch lies in two lines,
+// which the waves of its neighbours read as well, so the loads leave the lines in
+// the caches (complex m = n = 32, k = 4000001 1013 -> 812 us; 26 x 12, 6576433 791 ->
+// 687 us), and one fragment per operand takes two stretches at a time, three lines
+// for two (m = n = 16, k = 8000001 803 -> 678 us; more fragments have no registers
+// for it).
+bool rows_aligned(const GemmDesc& d, int elemBytes) {
+  const uint64_t bits = reinterpret_cast<uintptr_t>(d.A) | reinterpret_cast<uintptr_t>(d.B) |
+                        (d.m > 1 ? static_cast<uint64_t>(d.lda) * elemBytes : 0) |
+                        (d.n > 1 ? static_cast<uint64_t>(d.ldb) * elemBytes : 0);
+  return bits % kChunkRowBytes == 0;
+}
+
+template <bool CPLX, bool CONJ, int FM, int FN, int GROUPS = 1>
+hipError_t launch(const GemmDesc& d, hipStream_t stream) {
+  constexpr int kLines = GROUPS == 1 && FM == 1 && FN == 1 ? 2 : 1;
+  if (rows_aligned(d, CPLX ? 16 : 8))
+    hipLaunchKernelGGL((skinny_gemm_kernel<CPLX, CONJ, FM, FN, GROUPS, 1, true>), dim3(d.splits),
+                       dim3(kWaves * 64), 0, stream, d);
+  else
+    hipLaunchKernelGGL((skinny_gemm_kernel<CPLX, CONJ, FM, FN, GROUPS, kLines, false>),
+                       dim3(d.splits), dim3(kWaves * 64), 0, stream, d);
   return hipGetLastError();
 }
 
-template <bool CPLX>
+template <bool CPLX, bool CONJ>
 hipError_t launch_typed(const GemmDesc& d, hipStream_t stream) {
-  constexpr int ROWS = CPLX ? 8 : 16;
-  const int fm = d.m <= ROWS ? 1 : (d.m <= 2 * ROWS ? 2 : 4);
-  const int fn = d.n <= 16 ? 1 : 2;
-  if (fm == 1) return fn == 1 ? launch_fm_fn<CPLX, 1, 1>(d, stream) : launch_fm_fn<CPLX, 1, 2>(d, stream);
-  if (fm == 2) return fn == 1 ? launch_fm_fn<CPLX, 2, 1>(d, stream) : launch_fm_fn<CPLX, 2, 2>(d, stream);
-  return fn == 1 ? launch_fm_fn<CPLX, 4, 1>(d, stream) : launch_fm_fn<CPLX, 4, 2>(d, stream);
+  const bool wide = d.n > 16;
+  if (d.m > 32) {
+    if constexpr (!CPLX)
+      return wide ? launch<CPLX, CONJ, 4, 2>(d, stream) : launch<CPLX, CONJ, 4, 1>(d, stream);
+    return hipErrorInvalidValue;
+  }
+  if (d.m > 16)
+    return wide ? launch<CPLX, CONJ, 2, 2>(d, stream) : launch<CPLX, CONJ, 2, 1>(d, stream);
+  if (wide) return launch<CPLX, CONJ, 1, 2>(d, stream);
+  switch (skinny_groups(d.m, d.n)) {
+    case 16:
+      return launch<CPLX, CONJ, 1, 1, 16>(d, stream);
+    case 8:
+      return launch<CPLX, CONJ, 1, 1, 8>(d, stream);
+    case 4:
+      return launch<CPLX, CONJ, 1, 1, 4>(d, stream);
+    case 2:
+      return launch<CPLX, CONJ, 1, 1, 2>(d, stream);
+    default:
+      return launch<CPLX, CONJ, 1, 1>(d, stream);
+  }
 }
 
 }  // namespace
 
+int skinny_groups(int64_t m, int64_t n) {
+  const int64_t rows = m > n ? m : n;
+  return rows > 8 ? 1 : (rows > 4 ? 2 : (rows > 2 ? 4 : (rows > 1 ? 8 : 16)));
+}
+
 bool skinny_supported(bool complex, int layoutA, int layoutB, int64_t m, int64_t n) {
-  const int64_t rows = complex ? 8 : 16;
-  return layoutA == KMajor && layoutB == KMajor && m >= 1 && n >= 1 && m <= 4 * rows && n <= 32;
+  return layoutA == KMajor && layoutB == KMajor && m >= 1 && n >= 1 && m <= (complex ? 32 : 64) &&
+         n <= 32;
 }
 
 hipError_t launch_skinny_gemm(const GemmDesc& d, bool complex, hipStream_t stream) {
-  return complex ? launch_typed<true>(d, stream) : launch_typed<false>(d, stream);
+  if (!complex) return launch_typed<false, false>(d, stream);
+  return d.conjA != d.conjB ? launch_typed<true, true>(d, stream)
+                            : launch_typed<true, false>(d, stream);
 }
 
 }  // namespace spla_amd

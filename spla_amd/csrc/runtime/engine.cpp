@@ -127,13 +127,15 @@ struct Scalar<std::complex<float>> {
 
 // One product on device-resident operands, enqueued on `stream`. Workspace
 // blocks are appended to `keep` and must live until the stream is drained.
-// Skinny kernel: products with at least this embedded reduction length, split so
-// that every split holds at least kSkinnyMinKpPerSplit (16 steps per wave),
-// kSkinnyWgPerCU workgroups per CU.
+// Skinny kernel: products with at least this embedded reduction length, two
+// workgroups of four waves per CU (1024 partial results instead of 512 cost 2 to 5 %
+// at k = 8e6), fewer if their waves would not have two chunks of the reduction each.
 constexpr int64_t kSkinnyMinKp = 8192;
-constexpr int64_t kSkinnyMinKpPerSplit = 1024;
-constexpr int kSkinnyWgPerCU = 4;
-static_assert(kSkinnyMinKp >= 2 * kSkinnyMinKpPerSplit, "the skinny kernel writes split partials");
+constexpr int64_t kSkinnyChunkBytes = 128;
+constexpr int kSkinnyChunksPerWg = 8;
+constexpr int kSkinnyWgPerCU = 2;
+static_assert(kSkinnyMinKp * 8 >= 2 * 16 * kSkinnyChunkBytes * kSkinnyChunksPerWg,
+              "the skinny kernel writes split partials");
 
 // `fixed` (optional): caller-provided split-K workspace; nothing is allocated,
 // and a plan whose partial sums exceed it raises GPUAllocationError.
@@ -191,15 +193,14 @@ void enqueue_device_product(SplaOperation opA, SplaOperation opB, int64_t m, int
                        PlanFill{d.fillMode, d.fillRowOff, d.fillColOff});
   // Small m, n with a long reduction on a whole device: HBM-bound, streamed by
   // the skinny kernel (one workgroup per split, no LDS staging).
-  // (kSkinnyMinKp / kSkinnyMinKpPerSplit >= 2: always several splits)
+  // (at kSkinnyMinKp two workgroups have their chunks: always several splits)
   const bool skinny = !f32 && wholeChip && skinny_supported(cplx, la, lb, m, n) &&
                       d.Kp >= kSkinnyMinKp;
   if (skinny) {
-    const int64_t maxSplits = std::max<int64_t>(1, d.Kp / kSkinnyMinKpPerSplit);
-    int64_t sp = std::min<int64_t>(static_cast<int64_t>(ctx.num_cus()) * kSkinnyWgPerCU, maxSplits);
-    const int64_t kSplit = (d.Kp + sp - 1) / sp;
-    plan.kSplit = (kSplit + 15) / 16 * 16;
-    plan.splits = static_cast<int>((d.Kp + plan.kSplit - 1) / plan.kSplit);
+    const int64_t chunks = d.Kp * 8 / (kSkinnyChunkBytes * skinny_groups(m, n));
+    plan.splits = static_cast<int>(std::min<int64_t>(
+        static_cast<int64_t>(ctx.num_cus()) * kSkinnyWgPerCU, chunks / kSkinnyChunksPerWg));
+    plan.kSplit = (d.Kp + plan.splits - 1) / plan.splits;  // not used by the kernel
     plan.cfg = TileM;  // tile grid of the reduction's fill predicate
     plan.tilesM = plan.tilesN = 1;
   }
