@@ -27,6 +27,11 @@ bool skinny_supported(bool complex, int layoutA, int layoutB, int64_t m, int64_t
 int skinny_groups(int64_t m, int64_t n);
 hipError_t launch_skinny_gemm(const GemmDesc& d, bool complex, hipStream_t stream);
 
+// Product too small for the tile kernels, in one launch (small.hip); d's tiles and
+// splits are not read (f32: d's pointers are floats).
+hipError_t launch_small_gemm(const GemmDesc& d, bool complex, int layoutA, int layoutB,
+                             hipStream_t stream, bool f32);
+
 // Fixed-order sum of d.splits partial results in d.work, then alpha / beta
 // (f32: the scalars of d are floats).
 hipError_t launch_splitk_reduce(const GemmDesc& d, bool complex, int cfg, hipStream_t stream,

@@ -210,6 +210,11 @@ void enqueue_device_product(SplaOperation opA, SplaOperation opB, int64_t m, int
                                  fill, plan.estSeconds, stream, keep, reuse))
       return;
   }
+  if (plan.small) {
+    PhaseScope ps(ctx.timer(), PhaseGemmF64, stream);
+    hip_check(launch_small_gemm(d, cplx, la, lb, stream, f32));
+    return;
+  }
   d.splits = plan.splits;
   d.kSplit = plan.kSplit;
   d.tilesM = plan.tilesM;

@@ -126,6 +126,20 @@ GemmPlan plan_coarse(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, 
 constexpr double kSmallWorkspace = 64.0 * (1 << 20);
 constexpr double kLargestWorkspace = 256.0 * (1 << 20);
 
+// Products that one launch of 16 x 16 tiles (small.hip) does in less time than the tile
+// kernels. Its waves hold 512 reduction indices in flight, and every tile reads its rows
+// of A and B anew. Measured, us a call, tile kernels / small (launch and wait alone are
+// 15.6): d 13 x 32 x 263 24.4 / 17.2, 256 x 256 x 1024 27.1 / 22.4, 512 x 512 x 263 29.3 /
+// 21.4, but 13 x 32 x 2048 27.3 / 26.9 (A^T B 26.8 / 28.7) and 512 x 512 x 512 A^T B 28.1 /
+// 31.3; z 256 x 256 x 512 31.0 / 25.9, 1024 x 1024 x 32 A^H B 27.0 / 28.5; s 64 x 64 x 2048
+// 26.4 / 22.2, 1024 x 1024 x 32 20.4 / 21.3.
+bool small_product(int64_t m, int64_t n, int64_t Kp, int scalarBytes) {
+  constexpr int64_t kRows = 16, kMostTiles = 2048, kMostWork = int64_t(1) << 18;
+  const int64_t tilesM = (m + kRows - 1) / kRows, tilesN = (n + kRows - 1) / kRows;
+  if (tilesM > kMostTiles || tilesN > kMostTiles || tilesM * tilesN > kMostTiles) return false;
+  return Kp <= 8192 / scalarBytes && tilesM * tilesN * Kp <= kMostWork;
+}
+
 }  // namespace
 
 int64_t plan_active_tiles(int64_t m, int64_t n, int rows, int cols, const PlanFill& fill) {
@@ -167,6 +181,7 @@ GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, in
   const double limit = small ? kSmallWorkspace : kLargestWorkspace;
   const double bytes = static_cast<double>(m + n) * k * scalarBytes * (complex ? 2 : 1);
   GemmPlan best = coarse;
+  best.small = small_product(m, n, Kp, scalarBytes);
   double bestSeconds = 1e300, fullSeconds = 1e300;
   for (int cfg : {TileL, TileM}) {
     const TileShape ts = tile_shape(cfg);

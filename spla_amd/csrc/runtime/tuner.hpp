@@ -24,6 +24,7 @@ struct GemmPlan {
   int64_t kSplit = 0;   // embedded reduction length per split
   int tilesM = 0, tilesN = 0;
   double estSeconds = 0.0;
+  bool small = false;   // one launch of small.hip instead of the tiles above
 };
 
 // Part of C that a product needs (the kernels' TileFill and offsets).
