@@ -49,16 +49,18 @@ __device__ __forceinline__ void update_c(const BatchDesc& d, const BatchBlock& b
 }
 
 // Wave tiles of a configuration (see gemm_f64.hip): R = fragments per 32 embedded rows.
-template <bool CPLX, bool CONJ, int LA, int CFG, bool WIDE = false>
+// HALF: half of the columns (tiles of which no more exist, see gemm_tile).
+template <bool CPLX, bool CONJ, int LA, int CFG, bool HALF = false, bool WIDE = false>
 using BatchMma = TileMma<double, CPLX, CONJ, LA, KMajor, (CPLX ? 1 : 2) * (CFG == TileM ? 1 : 2),
-                         CFG == TileM ? 2 : 4, WIDE>;
+                         (CFG == TileM ? 2 : 4) / (HALF ? 2 : 1), WIDE>;
 
 // One (block, tile, split) item, its tile covered by repM x repN tiles of T; on
 // return every thread has passed the tile routine's last barrier, so the LDS
 // buffers may be reused at once.
-template <typename T, bool CPLX>
+template <typename T, typename H, bool CPLX>
 __device__ __forceinline__ void batched_item(const BatchDesc& d, const BatchItem& it, int repM,
-                                             int repN, typename T::Smem& sm) {
+                                             int repN, void* lds) {
+  static_assert(2 * H::BN == T::BN && H::AR == T::AR, "half of the columns");
   const BatchBlock& b = d.blocks[uniform(it.block)];
   const int m = uniform(b.m), n = uniform(b.n), Mp = uniform(b.Mp), s = uniform(it.s);
   const int64_t kSplit = uniform(b.kSplit);
@@ -71,21 +73,28 @@ __device__ __forceinline__ void batched_item(const BatchDesc& d, const BatchItem
   const bool flip = T::flip_result(d.conjA, d.conjB);
   const bool whole = uniform(b.splits) == 1;
   double* w = d.work + uniform(b.workOffset) + static_cast<int64_t>(s) * n * Mp;
+  auto run = [&](auto tile, int row, int col) {
+    using U = typename decltype(tile)::type;
+    typename U::Acc acc;
+    U::run(op, row, col, kBegin, kEnd, *static_cast<typename U::Smem*>(lds), acc);
+    if (whole) {
+      U::for_each(row, col, m, n, flip, acc,
+                  [&](int i, int j, double re, double im) { update_c<CPLX>(d, c, i, j, re, im); });
+    } else {
+      U::for_each(row, col, m, n, flip, acc, [&](int i, int j, double re, double im) {
+        store_work<double, CPLX>(w, Mp, i, j, re, im);
+      });
+    }
+  };
 #pragma unroll 1
   for (int t = 0; t < repM * repN; ++t) {
     const int row = (uniform(it.tm) * repM + t % repM) * T::AR;
     const int col = (uniform(it.tn) * repN + t / repM) * T::BN;
     if (row >= m || col >= n) continue;
-    typename T::Acc acc;
-    T::run(op, row, col, kBegin, kEnd, sm, acc);
-    if (whole) {
-      T::for_each(row, col, m, n, flip, acc,
-                  [&](int i, int j, double re, double im) { update_c<CPLX>(d, c, i, j, re, im); });
-    } else {
-      T::for_each(row, col, m, n, flip, acc, [&](int i, int j, double re, double im) {
-        store_work<double, CPLX>(w, Mp, i, j, re, im);
-      });
-    }
+    if (n - col <= H::BN)
+      run(Type<H>(), row, col);
+    else
+      run(Type<T>(), row, col);
   }
 }
 
@@ -93,17 +102,19 @@ __device__ __forceinline__ void batched_item(const BatchDesc& d, const BatchItem
 template <bool CPLX, bool CONJ, int LA, int CFG>
 __global__ void __launch_bounds__(kThreads, CFG == TileM ? 4 : 2) batched_gemm_kernel(BatchDesc d) {
   using T = BatchMma<CPLX, CONJ, LA, CFG>;
+  using H = BatchMma<CPLX, CONJ, LA, CFG, true>;
   __shared__ typename T::Smem sm;
-  batched_item<T, CPLX>(d, d.items[blockIdx.x], 1, 1, sm);
+  batched_item<T, H, CPLX>(d, d.items[blockIdx.x], 1, 1, &sm);
 }
 
 // The grouped launch for blocks with wide rows (tile_wide): every tile as M tiles.
 template <bool CPLX, bool CONJ, int LA, int CFG>
 __global__ void __launch_bounds__(kThreads, 2) batched_gemm_wide_kernel(BatchDesc d) {
-  using T = BatchMma<CPLX, CONJ, LA, TileM, true>;
+  using T = BatchMma<CPLX, CONJ, LA, TileM, false, true>;
+  using H = BatchMma<CPLX, CONJ, LA, TileM, true, true>;
   __shared__ typename T::Smem sm;
   constexpr int REP = CFG == TileM ? 1 : 2;
-  batched_item<T, CPLX>(d, d.items[blockIdx.x], REP, REP, sm);
+  batched_item<T, H, CPLX>(d, d.items[blockIdx.x], REP, REP, &sm);
 }
 
 // Persistent launch: one workgroup per slot works through its static list of
@@ -112,10 +123,11 @@ template <bool CPLX, bool CONJ, int LA, int CFG>
 __global__ void __launch_bounds__(kThreads, CFG == TileM ? 4 : 2)
     batched_gemm_persistent_kernel(BatchDesc d) {
   using T = BatchMma<CPLX, CONJ, LA, CFG>;
+  using H = BatchMma<CPLX, CONJ, LA, CFG, true>;
   __shared__ typename T::Smem sm;
   const int end = d.slotStart[blockIdx.x + 1];
   for (int i = d.slotStart[blockIdx.x]; i < end; ++i)
-    batched_item<T, CPLX>(d, d.items[uniform(d.slotItems[i])], 1, 1, sm);
+    batched_item<T, H, CPLX>(d, d.items[uniform(d.slotItems[i])], 1, 1, &sm);
 }
 
 // AR x BN: element rows and columns of a tile of the GEMM launch.

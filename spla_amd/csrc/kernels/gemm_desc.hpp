@@ -40,6 +40,7 @@ struct GemmDesc {
   int64_t kSplit; // embedded reduction length handled by one split (multiple of the k-block)
   int splits;
   int tilesM, tilesN;
+  int activeTiles;  // tiles that the fill mode needs (all of them without one)
 
   double alphaRe, alphaIm, betaRe, betaIm;
   int betaZero;  // beta == 0: C is written without being read

@@ -95,6 +95,11 @@ struct Index {
   static constexpr int value = N;
 };
 
+template <typename T>
+struct Type {
+  using type = T;
+};
+
 // The same value in a scalar register: loads through pointers that the kernel's
 // own stores might alias leave wave-uniform values in vector registers.
 template <typename V>
@@ -596,12 +601,6 @@ __device__ __forceinline__ void store_work(S* w, int64_t Mp, int i, int j, S re,
   S* p = w + static_cast<int64_t>(j) * Mp + (CPLX ? 2 * i : i);
   p[0] = re;
   if (CPLX) p[1] = im;
-}
-
-__device__ __forceinline__ double flip_sign(double x, uint32_t hiMask) {
-  uint64_t b = __builtin_bit_cast(uint64_t, x);
-  b ^= static_cast<uint64_t>(hiMask) << 32;
-  return __builtin_bit_cast(double, b);
 }
 
 }  // namespace tile

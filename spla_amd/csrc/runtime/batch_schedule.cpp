@@ -51,6 +51,7 @@ BatchSchedule plan_batch_schedule(const std::vector<BatchShape>& shapes, bool co
 
   struct Tile {
     int block, tm, tn;
+    double share;  // of the tile's cost: a half for the half tiles of batched.hip
   };
   std::vector<Tile> tiles;
   std::vector<double> tileCost(shapes.size(), 0.0);
@@ -68,8 +69,9 @@ BatchSchedule plan_batch_schedule(const std::vector<BatchShape>& shapes, bool co
         if (!batch_tile_active(s.fillMode, s.rowOff, s.colOff, r, c, std::min<int64_t>(ar, s.m - r),
                                std::min<int64_t>(ts.bn, s.n - c)))
           continue;
-        tiles.push_back({static_cast<int>(b), static_cast<int>(tm), static_cast<int>(tn)});
-        total += tileCost[b];
+        const double share = s.n - c <= ts.bn / 2 ? 0.5 : 1.0;
+        tiles.push_back({static_cast<int>(b), static_cast<int>(tm), static_cast<int>(tn), share});
+        total += share * tileCost[b];
       }
   }
   const double target = std::max(total / (3.0 * slots), 20e-6);
@@ -108,7 +110,8 @@ BatchSchedule plan_batch_schedule(const std::vector<BatchShape>& shapes, bool co
   for (const Tile& t : tiles) {
     const BatchBlock& bb = out.blocks[t.block];
     for (int q = 0; q < bb.splits; ++q)
-      items.push_back({{t.block, t.tm, t.tn, q}, tileCost[t.block] / bb.splits + kItemOverhead});
+      items.push_back({{t.block, t.tm, t.tn, q},
+                       t.share * tileCost[t.block] / bb.splits + kItemOverhead});
     if (bb.splits > 1) {
       out.reduce.push_back({t.block, t.tm, t.tn});
       reduceSeconds +=

@@ -215,10 +215,12 @@ void enqueue_device_product(SplaOperation opA, SplaOperation opB, int64_t m, int
     hip_check(launch_small_gemm(d, cplx, la, lb, stream, f32));
     return;
   }
+  if (plan.activeTiles == 0) return;  // no tile of C is needed
   d.splits = plan.splits;
   d.kSplit = plan.kSplit;
   d.tilesM = plan.tilesM;
   d.tilesN = plan.tilesN;
+  d.activeTiles = plan.activeTiles;
   if (plan.splits > 1) {
     const std::size_t bytes =
         static_cast<std::size_t>(plan.splits) * static_cast<std::size_t>(n) * d.Mp *

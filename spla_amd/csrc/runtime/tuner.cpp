@@ -163,22 +163,30 @@ int64_t plan_active_tiles(int64_t m, int64_t n, int rows, int cols, const PlanFi
 // CU reaches (700 x 700 x 30011 complex on M tiles: 242 workgroups 1.82 ms, 726
 // 1.72 ms). Past that the dispatcher hands workgroups out as slots free up, and a
 // last, partial round can land more than once on the same CU (1210 workgroups:
-// 2.07 ms), which many short rounds avoid (5808: 1.68 ms). Splitting the
-// reduction costs the write and read of the partial sums and a launch.
-GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, int forceCfg,
-                   int forceSplits, const double* effByCfg, bool wholeChip, int scalarBytes,
-                   const PlanFill& fill) {
+// 2.07 ms), which many short rounds avoid (5808: 1.68 ms; its lower triangle: 924
+// workgroups 1.00 ms, 4092 0.95 ms). Workgroups that start together do not end
+// together either (1000 x 1000 x 1e5 real on L tiles: 512 workgroups 3.00 ms, 1024
+// 2.94 ms). Splitting the reduction costs the write and read of the partial sums and
+// a launch.
+static GemmPlan plan_tiles(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, int forceCfg,
+                           int forceSplits, const double* effByCfg, bool wholeChip,
+                           int scalarBytes, const PlanFill& fill) {
   const GemmPlan coarse =
       plan_coarse(complex, m, n, k, numCUs, forceCfg, forceSplits, wholeChip);
   if (!wholeChip || forceCfg >= 0 || forceSplits > 0) return coarse;
   constexpr double kWorkgroupSeconds = 2.5e-6;  // address set-up, first loads, epilogue
   constexpr double kBlockSeconds = 0.6e-6;  // shortest k-block of one workgroup (latency)
+  constexpr double kLastRound = 0.03;  // of the last round: workgroups that finish apart
   constexpr double kReduceLaunchSeconds = 4.0e-6;
   const int64_t Mp = complex ? 2 * m : m;
   const int64_t Kp = complex ? 2 * k : k;
   const double sums = static_cast<double>(Mp) * n * scalarBytes;  // bytes of one split
-  const bool small = complex && scalarBytes == 8 && coarse.splits * sums <= kSmallWorkspace;
-  const double limit = small ? kSmallWorkspace : kLargestWorkspace;
+  const bool small = complex && scalarBytes == 8 && fill.mode == FillFull &&
+                     coarse.splits * sums <= kSmallWorkspace;
+  const double limit = small ? kSmallWorkspace
+                       : scalarBytes == 4
+                           ? std::max(kLargestWorkspace, coarse.splits * sums + 1)
+                           : kLargestWorkspace;
   const double bytes = static_cast<double>(m + n) * k * scalarBytes * (complex ? 2 : 1);
   GemmPlan best = coarse;
   best.small = small_product(m, n, Kp, scalarBytes);
@@ -190,13 +198,17 @@ GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, in
     const int64_t tilesM = (m + rows - 1) / rows, tilesN = (n + ts.bn - 1) / ts.bn;
     const int64_t allTiles = tilesM * tilesN;
     const int64_t tiles = std::max<int64_t>(1, plan_active_tiles(m, n, rows, ts.bn, fill));
+    // half tiles at the right edge and along the diagonal of a fill mode cost half
+    const double share = std::min(
+        1.0, 0.5 * plan_active_tiles(m, n, rows, ts.bn / 2, fill) / static_cast<double>(tiles));
+    const double needed = static_cast<double>(tiles) / allTiles;  // of C
     const int64_t kBlocks = std::max<int64_t>(1, (Kp + bk - 1) / bk);
     const int perCU = blocks_per_cu(cfg);
     const int64_t slots = static_cast<int64_t>(numCUs) * perCU;
     const double peak = kPeakPerCU * (8.0 / scalarBytes) * effByCfg[cfg];
     const double lone = cfg == TileL ? 0.85 : 0.88;
     const int64_t maxSplits = std::max<int64_t>(
-        1, std::min<int64_t>(kBlocks / 8, std::max<int64_t>(64, 4 * slots / tiles)));
+        1, std::min<int64_t>(kBlocks / scalarBytes, std::max<int64_t>(64, 4 * slots / tiles)));
     int64_t lastSplits = 0;
     for (int64_t s = 1; s <= maxSplits; s += std::max<int64_t>(1, s / 32)) {
       const int64_t kb = (kBlocks + s - 1) / s;
@@ -204,20 +216,25 @@ GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, in
       if (splits == lastSplits || allTiles * splits > (int64_t(1) << 31) - 1) continue;
       lastSplits = splits;
       if (splits > 1 && splits * sums > limit) break;
+      // single precision: no longer sums than the coarse plan's, since their rounding
+      // errors grow with the length (s 4 x 10 x 309: 1.9e-7 of the result in 2 splits,
+      // 2.9e-7 in 1)
+      if (scalarBytes == 4 && kb * bk >= coarse.kSplit + bk) continue;
       const double work = 2.0 * ts.bm * ts.bn * bk * kb / peak;  // one workgroup on a full CU
       auto seconds = [&](int64_t groups) {
         const int64_t rounds = groups / slots, rest = groups % slots;
-        double t = rounds * perCU * work + (rounds > 0 ? (0.7 + 0.3 * rounds) : 0.0) *
+        double t = rounds * perCU * work * share + (rounds > 0 ? (0.7 + 0.3 * rounds) : 0.0) *
                                                kWorkgroupSeconds;
         if (rest > 0) {
           const int64_t spread = (rest + numCUs - 1) / numCUs;
           const int64_t q = rounds > 0 ? std::min<int64_t>(perCU, spread + 1) : spread;
           t += std::max(q * work / (q == 1 ? lone : 1.0), kb * kBlockSeconds) + kWorkgroupSeconds;
         }
+        t += kLastRound * work * std::min<double>(perCU, groups / static_cast<double>(numCUs));
         const double inFlight = std::min(1.0, groups / (2.0 * numCUs));
         t = std::max(t, bytes / (kHbmBytesPerSecond * inFlight)) + kLaunchSeconds;
         if (splits > 1)
-          t += (1.5 * splits + 2) * sums / kHbmBytesPerSecond + kReduceLaunchSeconds;
+          t += (1.2 * splits + 2) * sums * needed / kHbmBytesPerSecond + kReduceLaunchSeconds;
         return t;
       };
       const double t = seconds(tiles * splits);
@@ -236,6 +253,17 @@ GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, in
   // drawn for the coarse model's rates, 0.84 of those reached now
   best.estSeconds = std::min(coarse.estSeconds, fullSeconds / 0.84);
   return best;
+}
+
+GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, int forceCfg,
+                   int forceSplits, const double* effByCfg, bool wholeChip, int scalarBytes,
+                   const PlanFill& fill) {
+  GemmPlan p = plan_tiles(complex, m, n, k, numCUs, forceCfg, forceSplits, effByCfg, wholeChip,
+                          scalarBytes, fill);
+  const TileShape ts = tile_shape(p.cfg);
+  p.activeTiles =
+      static_cast<int>(plan_active_tiles(m, n, complex ? ts.bm / 2 : ts.bm, ts.bn, fill));
+  return p;
 }
 
 // Measured on long reductions: 2048 x 2048 x 2e4, complex and real, 74.2-75.6

@@ -23,6 +23,7 @@ struct GemmPlan {
   int splits = 1;       // split-K factor
   int64_t kSplit = 0;   // embedded reduction length per split
   int tilesM = 0, tilesN = 0;
+  int activeTiles = 0;  // of these, the tiles that the fill mode needs
   double estSeconds = 0.0;
   bool small = false;   // one launch of small.hip instead of the tiles above
 };

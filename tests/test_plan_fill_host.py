@@ -4,7 +4,8 @@
 * the closed form of the active tiles equals SPLA's block_is_active
   (src/block_generation/block.hpp:58-66) counted tile by tile;
 * plans of every fill mode and scalar size cover the reduction in whole 128-byte
-  k-blocks with no empty split, and their partial sums stay within 256 MiB.
+  k-blocks with no empty split; double partial sums stay within 256 MiB (single
+  precision may take more, to keep its sums short).
 """
 
 import ctypes
@@ -72,5 +73,5 @@ def test_plans_cover_the_reduction(lib, cplx, scalar):
                     kp = k * (1 + cplx)
                     assert per > 0 and per % unit == 0 and tm > 0 and tn > 0
                     assert splits * per >= kp and (splits - 1) * per < kp
-                    if splits > 1:
+                    if splits > 1 and scalar == 8:
                         assert splits * n * m * (1 + cplx) * scalar <= 256 << 20
