@@ -18,9 +18,11 @@ __device__ __forceinline__ bool tile_active(const GemmDesc& d, int64_t r, int64_
   return true;
 }
 
-// C <- alpha * (re, im) + beta * C in the scalar type S (beta == 0: C not read).
+// C <- alpha * (re, im) + beta * (cr, ci) in the scalar type S; (cr, ci): C before, not
+// used when beta == 0.
 template <typename S, bool CPLX>
-__device__ __forceinline__ void store_result(const GemmDesc& d, int i, int j, S re, S im) {
+__device__ __forceinline__ void store_update(const GemmDesc& d, int i, int j, S re, S im, S cr,
+                                             S ci) {
   const S aRe = static_cast<S>(d.alphaRe), aIm = static_cast<S>(d.alphaIm);
   const S bRe = static_cast<S>(d.betaRe), bIm = static_cast<S>(d.betaIm);
   if (CPLX) {
@@ -28,7 +30,6 @@ __device__ __forceinline__ void store_result(const GemmDesc& d, int i, int j, S 
     S outRe = aRe * re - aIm * im;
     S outIm = aRe * im + aIm * re;
     if (!d.betaZero) {
-      const S cr = c[0], ci = c[1];
       outRe += bRe * cr - bIm * ci;
       outIm += bRe * ci + bIm * cr;
     }
@@ -36,10 +37,22 @@ __device__ __forceinline__ void store_result(const GemmDesc& d, int i, int j, S 
     c[1] = outIm;
   } else {
     S* c = static_cast<S*>(d.C) + static_cast<int64_t>(j) * d.ldc + i;
-    S out = aRe * re;
-    if (!d.betaZero) out += bRe * c[0];
-    c[0] = out;
+    // written out: which product the compiler rounds first differs with its surroundings
+    const S out = aRe * re;
+    c[0] = d.betaZero ? out : static_cast<S>(fma(bRe, cr, out));
   }
+}
+
+// The same, reading C (beta == 0: C not read).
+template <typename S, bool CPLX>
+__device__ __forceinline__ void store_result(const GemmDesc& d, int i, int j, S re, S im) {
+  S cr = S(0), ci = S(0);
+  if (!d.betaZero) {
+    const S* c = static_cast<const S*>(d.C) + (static_cast<int64_t>(j) * d.ldc + i) * (CPLX ? 2 : 1);
+    cr = c[0];
+    if (CPLX) ci = c[1];
+  }
+  store_update<S, CPLX>(d, i, j, re, im, cr, ci);
 }
 
 }  // namespace spla_amd

@@ -115,9 +115,15 @@ __device__ __forceinline__ void gemm_tile(const GemmDesc& d, int repM, int repN,
     if (d.splits > 1) {
       U::for_each(row, col, d.m, d.n, flip, acc,
                   [&](int i, int j, S re, S im) { store_work<S, CPLX>(w, d.Mp, i, j, re, im); });
+    } else if (d.betaZero) {
+      U::for_each(row, col, d.m, d.n, flip, acc, [&](int i, int j, S re, S im) {
+        store_update<S, CPLX>(d, i, j, re, im, S(0), S(0));
+      });
     } else {
-      U::for_each(row, col, d.m, d.n, flip, acc,
-                  [&](int i, int j, S re, S im) { store_result<S, CPLX>(d, i, j, re, im); });
+      U::for_each_update(row, col, d.m, d.n, flip, acc, static_cast<const S*>(d.C), d.ldc,
+                         [&](int i, int j, S re, S im, S cr, S ci) {
+                           store_update<S, CPLX>(d, i, j, re, im, cr, ci);
+                         });
     }
   };
   auto one = [&](int row, int col) {

@@ -174,7 +174,6 @@ static GemmPlan plan_tiles(bool complex, int64_t m, int64_t n, int64_t k, int nu
   const GemmPlan coarse =
       plan_coarse(complex, m, n, k, numCUs, forceCfg, forceSplits, wholeChip);
   if (!wholeChip || forceCfg >= 0 || forceSplits > 0) return coarse;
-  constexpr double kWorkgroupSeconds = 2.5e-6;  // address set-up, first loads, epilogue
   constexpr double kBlockSeconds = 0.6e-6;  // shortest k-block of one workgroup (latency)
   constexpr double kLastRound = 0.03;  // of the last round: workgroups that finish apart
   constexpr double kReduceLaunchSeconds = 4.0e-6;
@@ -207,6 +206,9 @@ static GemmPlan plan_tiles(bool complex, int64_t m, int64_t n, int64_t k, int nu
     const int64_t slots = static_cast<int64_t>(numCUs) * perCU;
     const double peak = kPeakPerCU * (8.0 / scalarBytes) * effByCfg[cfg];
     const double lone = cfg == TileL ? 0.85 : 0.88;
+    // address set-up, first loads, epilogue (complex 60000 x 128 x 128: 142 us on M tiles,
+    // 164 us on L tiles, which the same time for both preferred)
+    const double workgroupSeconds = cfg == TileL ? 10e-6 : 2.5e-6;
     const int64_t maxSplits = std::max<int64_t>(
         1, std::min<int64_t>(kBlocks / scalarBytes, std::max<int64_t>(64, 4 * slots / tiles)));
     int64_t lastSplits = 0;
@@ -224,11 +226,11 @@ static GemmPlan plan_tiles(bool complex, int64_t m, int64_t n, int64_t k, int nu
       auto seconds = [&](int64_t groups) {
         const int64_t rounds = groups / slots, rest = groups % slots;
         double t = rounds * perCU * work * share + (rounds > 0 ? (0.7 + 0.3 * rounds) : 0.0) *
-                                               kWorkgroupSeconds;
+                                               workgroupSeconds;
         if (rest > 0) {
           const int64_t spread = (rest + numCUs - 1) / numCUs;
           const int64_t q = rounds > 0 ? std::min<int64_t>(perCU, spread + 1) : spread;
-          t += std::max(q * work / (q == 1 ? lone : 1.0), kb * kBlockSeconds) + kWorkgroupSeconds;
+          t += std::max(q * work / (q == 1 ? lone : 1.0), kb * kBlockSeconds) + workgroupSeconds;
         }
         t += kLastRound * work * std::min<double>(perCU, groups / static_cast<double>(numCUs));
         const double inFlight = std::min(1.0, groups / (2.0 * numCUs));
