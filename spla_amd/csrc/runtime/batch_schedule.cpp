@@ -3,8 +3,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <functional>
-#include <queue>
 
 #include "kernels/gemm_desc.hpp"
 #include "spla/types.h"
@@ -101,48 +99,66 @@ BatchSchedule plan_batch_schedule(const std::vector<BatchShape>& shapes, bool co
     }
   }
 
+  // items in decreasing cost order: the splits of a tile cost the same, so the tiles are
+  // ordered and their splits follow each other
   struct Costed {
     BatchItem item;
     double cost;
   };
-  std::vector<Costed> items;
+  std::vector<std::pair<double, int>> order(tiles.size());  // (cost of a split, tile)
+  std::size_t count = 0;
   double reduceSeconds = 0.0;
-  for (const Tile& t : tiles) {
+  for (std::size_t i = 0; i < tiles.size(); ++i) {
+    const Tile& t = tiles[i];
     const BatchBlock& bb = out.blocks[t.block];
-    for (int q = 0; q < bb.splits; ++q)
-      items.push_back({{t.block, t.tm, t.tn, q},
-                       t.share * tileCost[t.block] / bb.splits + kItemOverhead});
+    order[i] = {t.share * tileCost[t.block] / bb.splits + kItemOverhead, static_cast<int>(i)};
+    count += bb.splits;
     if (bb.splits > 1) {
       out.reduce.push_back({t.block, t.tm, t.tn});
       reduceSeconds +=
           (bb.splits + 2.0) * ar * ts.bn * 8.0 * comps / kReduceBytesPerSecond;
     }
   }
-  std::stable_sort(items.begin(), items.end(),
-                   [](const Costed& a, const Costed& b) { return a.cost > b.cost; });
+  std::stable_sort(order.begin(), order.end(),
+                   [](const auto& a, const auto& b) { return a.first > b.first; });
+  std::vector<Costed> items;
+  items.reserve(count);
+  for (const auto& o : order) {
+    const Tile& t = tiles[o.second];
+    for (int q = 0; q < out.blocks[t.block].splits; ++q)
+      items.push_back({{t.block, t.tm, t.tn, q}, o.first});
+  }
   out.items.reserve(items.size());
   // longest processing time first: each item goes to the slot that frees up
   // first (ties: the lowest slot), which is also the persistent launch's schedule
   const int nSlots = batch_slots(cfg, numCUs, items.size());
   using Slot = std::pair<double, int>;  // (load, slot)
-  std::priority_queue<Slot, std::vector<Slot>, std::greater<Slot>> load;
-  for (int i = 0; i < nSlots; ++i) load.push({0.0, i});
-  std::vector<std::vector<int>> perSlot(nSlots);
+  std::vector<Slot> load(nSlots);  // a heap, the least load first
+  for (int i = 0; i < nSlots; ++i) load[i] = {0.0, i};
+  std::vector<int> slotOf(items.size());
+  out.slotStart.assign(nSlots + 1, 0);
   double makespan = 0.0;
   for (std::size_t i = 0; i < items.size(); ++i) {
     out.items.push_back(items[i].item);
-    Slot sl = load.top();
-    load.pop();
+    Slot sl = load[0];
     sl.first += items[i].cost;
     makespan = std::max(makespan, sl.first);
-    perSlot[sl.second].push_back(static_cast<int>(i));
-    load.push(sl);
+    slotOf[i] = sl.second;
+    ++out.slotStart[sl.second + 1];
+    int at = 0;  // the slot sinks to its new place
+    for (int child = 1; child < nSlots; child = 2 * at + 1) {
+      if (child + 1 < nSlots && load[child + 1] < load[child]) ++child;
+      if (!(load[child] < sl)) break;
+      load[at] = load[child];
+      at = child;
+    }
+    load[at] = sl;
   }
-  out.slotStart.assign(1, 0);
-  for (const std::vector<int>& v : perSlot) {
-    out.slotItems.insert(out.slotItems.end(), v.begin(), v.end());
-    out.slotStart.push_back(static_cast<int>(out.slotItems.size()));
-  }
+  for (int w = 0; w < nSlots; ++w) out.slotStart[w + 1] += out.slotStart[w];
+  out.slotItems.resize(items.size());
+  std::vector<int> next(out.slotStart.begin(), out.slotStart.end() - 1);
+  for (std::size_t i = 0; i < items.size(); ++i)
+    out.slotItems[next[slotOf[i]]++] = static_cast<int>(i);
   out.modelSeconds = makespan + reduceSeconds + kLaunchOverhead * (out.reduce.empty() ? 1 : 2);
   return out;
 }
