@@ -42,9 +42,8 @@ int env_tile() {
   return -1;
 }
 
-// Plan and time of a coarse model that the forced plans, the block products of a
-// batch and the automatic mode's choice of arithmetic are made with: waves of
-// workgroups over the resident slots, no fill mode.
+}  // namespace
+
 GemmPlan plan_coarse(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, int forceCfg,
                      int forceSplits, bool wholeChip) {
   const int64_t Mp = complex ? 2 * m : m;
@@ -121,8 +120,10 @@ GemmPlan plan_coarse(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, 
   return best;
 }
 
+namespace {
+
 // Bytes of partial sums. The allocation-free entry point (complex doubles) holds
-// 64 MiB: a product whose coarse plan fits keeps within it.
+// 64 MiB: a product whose coarse plan fits, with one split too, keeps within it.
 constexpr double kSmallWorkspace = 64.0 * (1 << 20);
 constexpr double kLargestWorkspace = 256.0 * (1 << 20);
 
@@ -181,7 +182,7 @@ static GemmPlan plan_tiles(bool complex, int64_t m, int64_t n, int64_t k, int nu
   const int64_t Kp = complex ? 2 * k : k;
   const double sums = static_cast<double>(Mp) * n * scalarBytes;  // bytes of one split
   const bool small = complex && scalarBytes == 8 && fill.mode == FillFull &&
-                     coarse.splits * sums <= kSmallWorkspace;
+                     (coarse.splits == 1 || coarse.splits * sums <= kSmallWorkspace);
   const double limit = small ? kSmallWorkspace
                        : scalarBytes == 4
                            ? std::max(kLargestWorkspace, coarse.splits * sums + 1)

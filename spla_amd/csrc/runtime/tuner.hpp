@@ -58,6 +58,13 @@ private:
 // tile_active over all tiles of an m x n matrix).
 int64_t plan_active_tiles(int64_t m, int64_t n, int rows, int cols, const PlanFill& fill);
 
+// Plan and time of a coarse model that the forced plans, the block products of a
+// batch and the automatic mode's choice of arithmetic are made with: waves of
+// workgroups over the resident slots, no fill mode. Its split count also says which
+// products the allocation-free entry point takes.
+GemmPlan plan_coarse(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, int forceCfg,
+                     int forceSplits, bool wholeChip);
+
 // Pure cost model (no state), exposed for tests.
 GemmPlan plan_gemm(bool complex, int64_t m, int64_t n, int64_t k, int numCUs, int forceCfg,
                    int forceSplits, const double* effByCfg, bool wholeChip = true,
