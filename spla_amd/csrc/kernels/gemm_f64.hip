@@ -21,6 +21,7 @@
 
 #include <cstdint>
 
+#include "kernels/fill_tiles.hpp"
 #include "kernels/gemm_desc.hpp"
 #include "kernels/gemm_epilogue.hpp"
 #include "kernels/launch.hpp"
@@ -30,21 +31,6 @@ namespace spla_amd {
 namespace {
 
 using namespace tile;
-
-// Tile rows [first, end) of tile column tn that the fill mode needs (tile_active over
-// tiles of rows x cols).
-__device__ __forceinline__ void active_rows(const GemmDesc& d, int rows, int cols, int tn,
-                                            int& first, int& end) {
-  const int64_t c = static_cast<int64_t>(tn) * cols + d.fillColOff - d.fillRowOff;
-  first = 0;
-  end = d.tilesM;
-  if (d.fillMode == FillUpper) {
-    const int64_t last = c + min(cols, d.n - tn * cols);  // tiles that begin above this row
-    end = last <= 0 ? 0 : static_cast<int>(min<int64_t>(d.tilesM, (last + rows - 1) / rows));
-  } else if (d.fillMode == FillLower) {
-    first = c <= 0 ? 0 : (c >= d.m ? d.tilesM : static_cast<int>(c / rows));
-  }
-}
 
 // Maps the workgroup index to (split, tile row, tile column) over the active tiles of
 // rows x cols. Only these are launched: workgroups that leave at once let the
@@ -57,16 +43,11 @@ __device__ __forceinline__ void map_block(const GemmDesc& d, int rows, int cols,
   int lin = bid;
   if ((G & 7) == 0) lin = (bid & 7) * (G >> 3) + (bid >> 3);
   s = lin / d.activeTiles;
-  int t = lin - s * d.activeTiles;
-  if (d.fillMode != FillFull) {
-    for (tn = 0; tn < d.tilesN; ++tn) {  // tile by tile down the columns
-      int first, end;
-      active_rows(d, rows, cols, tn, first, end);
-      tm = first + t;
-      if (t < end - first) return;
-      t -= max(0, end - first);
-    }
-    s = -1;  // not reached: the grid has the active tiles
+  const int t = lin - s * d.activeTiles;
+  if (d.fillMode != FillFull) {  // tile by tile down the columns
+    const FillTiles tiles{d.fillMode, d.fillColOff - d.fillRowOff, d.m, d.n, rows, cols,
+                          d.tilesM, d.tilesN};
+    tiles.locate(t, tm, tn);
     return;
   }
   constexpr int kGroup = 8;
@@ -90,7 +71,6 @@ __device__ __forceinline__ void gemm_tile(const GemmDesc& d, int repM, int repN,
   if (!MULTI) repM = repN = 1;
   int s, tm, tn;
   map_block(d, T::AR * repM, T::BN * repN, s, tm, tn);
-  if (s < 0) return;
   const int first = tm * T::AR * repM;
   const int col0 = tn * T::BN * repN;
   bool left = true, right = true;  // half tiles that are needed

@@ -6,6 +6,7 @@
 #include <cstring>
 #include <vector>
 
+#include "kernels/fill_tiles.hpp"
 #include "kernels/gemm_desc.hpp"
 
 namespace spla_amd {
@@ -146,16 +147,8 @@ bool small_product(int64_t m, int64_t n, int64_t Kp, int scalarBytes) {
 int64_t plan_active_tiles(int64_t m, int64_t n, int rows, int cols, const PlanFill& fill) {
   const int64_t tilesM = (m + rows - 1) / rows, tilesN = (n + cols - 1) / cols;
   if (fill.mode == FillFull) return tilesM * tilesN;
-  int64_t count = 0;
-  for (int64_t tn = 0; tn < tilesN; ++tn) {
-    const int64_t c = tn * cols + fill.colOff - fill.rowOff;
-    const int64_t nc = std::min<int64_t>(cols, n - tn * cols);
-    if (fill.mode == FillUpper)  // first row of the tile before the last column's diagonal entry
-      count += std::max<int64_t>(0, std::min(tilesM, (c + nc + rows - 1) / rows));
-    else if (c < m)  // last row of the tile past the first column's diagonal entry
-      count += tilesM - std::max<int64_t>(0, c) / rows;
-  }
-  return count;
+  if (tilesM <= 0 || tilesN <= 0) return 0;
+  return FillTiles{fill.mode, fill.colOff - fill.rowOff, m, n, rows, cols, tilesM, tilesN}.total();
 }
 
 // Whole-device plans. Every workgroup of a launch computes one tile over one
