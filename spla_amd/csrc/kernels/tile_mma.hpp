@@ -472,6 +472,11 @@ struct TileMma {
     // Small wave tiles load two k-blocks ahead through two register sets, the
     // larger ones one and a half (k-block it + 2 as soon as it + 1 is stored).
     constexpr bool kTwoAhead = FM * FN * kComps <= 4;
+    // Left to itself the compiler begins a k-block's loads between the stores of the one in
+    // front, for which the large real double tiles with one MN-major operand lack the
+    // registers: 5 spilled, two of them read back in the loop (2048 x 2048 x 2e4 A B 2.50
+    // ms, 2.39 with the loads last). The others have them and lose 1 % with the loads last.
+    constexpr bool kLoadsLast = kF64 && !CPLX && LA != LB;
     typename StageA::Regs ra[kTwoAhead ? 2 : 1];
     typename StageB::Regs rb[kTwoAhead ? 2 : 1];
     FragsA fa[2];
@@ -528,7 +533,10 @@ struct TileMma {
       __builtin_amdgcn_sched_barrier(0);
       StageA::store(ra[kStored], sm.a[CUR ^ 1]);
       StageB::store(rb[kStored], sm.b[CUR ^ 1]);
-      if (!kTwoAhead && !kTail) next(0);
+      if (!kTwoAhead && !kTail) {
+        if constexpr (kLoadsLast) __builtin_amdgcn_sched_barrier(0);
+        next(0);
+      }
 #pragma unroll
       for (int p = kPasses / 2; p < kPasses; ++p) mfma_pass(acc, fa[0], fb[0], p);
       __builtin_amdgcn_sched_barrier(0);  // these MFMAs cover the stores' completion
