@@ -38,6 +38,8 @@ struct GemmDesc {
   int Mp;         // embedded output rows: m (real) or 2m (complex)
   int64_t Kp;     // embedded reduction length: k (real) or 2k (complex)
   int64_t kSplit; // embedded reduction length handled by one split (multiple of the k-block)
+  int64_t kSum;   // 0, or the embedded length summed at a time (two k-blocks or a multiple):
+                  // the sums of a split are added up (TileM, double precision)
   int splits;
   int tilesM, tilesN;
   int activeTiles;  // tiles that the fill mode needs (all of them without one)

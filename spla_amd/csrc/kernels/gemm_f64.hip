@@ -65,12 +65,16 @@ __device__ __forceinline__ void map_block(const GemmDesc& d, int rows, int cols,
 // half tile H: the matrix cores are what bounds the kernel, so the other half is not
 // computed (real 100003 x 260 x 260 341 -> 326 us, a batch of 128 ragged complex blocks 14.1
 // -> 13.7 ms).
-template <typename T, typename H, typename S, bool CPLX, bool MULTI>
+// STRETCHES: see TileMma::run.
+template <typename T, typename H, typename S, bool CPLX, bool MULTI, bool STRETCHES = false>
 __device__ __forceinline__ void gemm_tile(const GemmDesc& d, int repM, int repN, void* lds) {
   static_assert(2 * H::BN == T::BN && H::AR == T::AR, "half of the columns");
   if (!MULTI) repM = repN = 1;
   int s, tm, tn;
   map_block(d, T::AR * repM, T::BN * repN, s, tm, tn);
+  s = uniform(s);
+  tm = uniform(tm);
+  tn = uniform(tn);
   const int first = tm * T::AR * repM;
   const int col0 = tn * T::BN * repN;
   bool left = true, right = true;  // half tiles that are needed
@@ -88,10 +92,13 @@ __device__ __forceinline__ void gemm_tile(const GemmDesc& d, int repM, int repN,
                            uniform(d.lda), uniform(d.ldb), uniform(d.m), uniform(d.n)};
   const bool flip = T::flip_result(d.conjA, d.conjB);
   S* w = static_cast<S*>(d.work) + static_cast<int64_t>(s) * d.n * d.Mp;
+  constexpr int kBlock = kBlockBytes / sizeof(S);  // embedded
+  const int stretch = d.kSum > 0 ? static_cast<int>(d.kSum / kBlock) : 1 << 30;
   auto run = [&](auto tile, int row, int col) {
     using U = typename decltype(tile)::type;
     typename U::Acc acc;
-    U::run(op, row, col, kBegin, kEnd, *static_cast<typename U::Smem*>(lds), acc);
+    U::template run<STRETCHES>(op, row, col, kBegin, kEnd, *static_cast<typename U::Smem*>(lds),
+                               acc, stretch);
     if (d.splits > 1) {
       U::for_each(row, col, d.m, d.n, flip, acc,
                   [&](int i, int j, S re, S im) { store_work<S, CPLX>(w, d.Mp, i, j, re, im); });
@@ -133,13 +140,27 @@ __global__ void __launch_bounds__(kThreads, MINBLOCKS) gemm_f64_kernel(GemmDesc 
   gemm_tile<T, H, double, CPLX, false>(d, 1, 1, &sm);
 }
 
+// M tiles that add their sums up in stretches (GemmDesc::kSum), so that a product needs
+// neither longer sums nor the memory traffic of more splits: complex 1238 x 1207 x 4119
+// 0.73 ms and 2.6e-14 root mean square error in one split; one long sum has 0.72 ms and
+// 1.3e-13, 28 splits on L tiles 1.09 ms and 2.6e-14. The totals fit beside the four
+// workgroups per CU of complex tiles; real ones have registers for three (1601 x 1190 x
+// 20905 1.28 ms either way).
+template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN>
+__global__ void __launch_bounds__(kThreads, CPLX ? 4 : 3) gemm_f64_stretch_kernel(GemmDesc d) {
+  using T = TileMma<double, CPLX, CONJ, LA, LB, FM, FN>;
+  using H = TileMma<double, CPLX, CONJ, LA, LB, FM, FN / 2>;
+  __shared__ typename T::Smem sm;
+  gemm_tile<T, H, double, CPLX, false, true>(d, 1, 1, &sm);
+}
+
 // Tiles of repM x repN of the kernel's own (see launch_layout).
 template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN, bool WIDE>
 __global__ void __launch_bounds__(kThreads, 2) gemm_f64_multi_kernel(GemmDesc d, int repM, int repN) {
   using T = TileMma<double, CPLX, CONJ, LA, LB, FM, FN, WIDE>;
   using H = TileMma<double, CPLX, CONJ, LA, LB, FM, FN / 2, WIDE>;
   __shared__ typename T::Smem sm;
-  gemm_tile<T, H, double, CPLX, true>(d, repM, repN, &sm);
+  gemm_tile<T, H, double, CPLX, true, WIDE>(d, repM, repN, &sm);
 }
 
 template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN, int MINBLOCKS>
@@ -300,8 +321,12 @@ hipError_t launch_layout(const GemmDesc& d, int cfg, hipStream_t stream) {
   } else {
     switch (cfg) {
       case TileM:
-        hipLaunchKernelGGL((gemm_f64_kernel<CPLX, CONJ, LA, LB, R, 2, 4>), grid, block, 0, stream,
-                           d);
+        if (d.kSum > 0)
+          hipLaunchKernelGGL((gemm_f64_stretch_kernel<CPLX, CONJ, LA, LB, R, 2>), grid, block, 0,
+                             stream, d);
+        else
+          hipLaunchKernelGGL((gemm_f64_kernel<CPLX, CONJ, LA, LB, R, 2, 4>), grid, block, 0,
+                             stream, d);
         break;
       case TileXL:
         hipLaunchKernelGGL((gemm_f64_multi_kernel<CPLX, CONJ, LA, LB, 2 * R, 4, false>), grid,

@@ -453,8 +453,36 @@ struct TileMma {
     }
   }
 
+  __device__ __forceinline__ static void clear(Acc& acc) {
+#pragma unroll
+    for (int f = 0; f < FM; ++f)
+#pragma unroll
+      for (int g = 0; g < FN; ++g) {
+        acc.re[f][g] = V4{S(0), S(0), S(0), S(0)};
+        if (CPLX) acc.im[f % (CPLX ? FM : 1)][g % (CPLX ? FN : 1)] = V4{S(0), S(0), S(0), S(0)};
+      }
+  }
+  // total += acc
+  __device__ __forceinline__ static void add(Acc& total, const Acc& acc) {
+#pragma unroll
+    for (int f = 0; f < FM; ++f)
+#pragma unroll
+      for (int g = 0; g < FN; ++g) {
+        total.re[f][g] += acc.re[f][g];
+        if (CPLX) {
+          constexpr int kM = CPLX ? FM : 1, kN = CPLX ? FN : 1;
+          total.im[f % kM][g % kN] += acc.im[f % kM][g % kN];
+        }
+      }
+  }
+
+  // STRETCHES: every `stretch` k-blocks (even, at least 2) the accumulators are added to
+  // totals and start anew, so that rounding errors grow with the length of a stretch and
+  // not of the whole range. The totals take as many registers again.
+  template <bool STRETCHES = false>
   __device__ __forceinline__ static void run(const TileOperands<S>& op, int row0, int col0,
-                                             int64_t kBegin, int64_t kEnd, Smem& sm, Acc& acc) {
+                                             int64_t kBegin, int64_t kEnd, Smem& sm, Acc& acc,
+                                             int stretch = 0) {
     const int wave = threadIdx.x >> 6;
     const int wa = (wave % WAVES_M) * 16 * FM;
     const int wb = (wave / WAVES_M) * 16 * FN;
@@ -500,14 +528,19 @@ struct TileMma {
         StageB::store(pb, sm.b[0]);
       }
     }
-#pragma unroll
-    for (int f = 0; f < FM; ++f)
-#pragma unroll
-      for (int g = 0; g < FN; ++g) {
-        acc.re[f][g] = V4{S(0), S(0), S(0), S(0)};
-        if (CPLX) acc.im[f % (CPLX ? FM : 1)][g % (CPLX ? FN : 1)] = V4{S(0), S(0), S(0), S(0)};
-      }
+    clear(acc);
     if (nk == 0) return;
+    Acc total;
+    if constexpr (STRETCHES) clear(total);
+    int edge = stretch;  // k-blocks in front of the next stretch
+    auto stretch_end = [&](int done) {
+      if constexpr (STRETCHES) {
+        if (done != edge) return;
+        add(total, acc);
+        clear(acc);
+        edge += stretch;
+      }
+    };
     __syncthreads();
     fa[0].read(sm.a[0], wa, 0);
     fb[0].read(sm.b[0], wb, 0);
@@ -561,6 +594,7 @@ struct TileMma {
       };
       kblock(Index<0>(), Index<0>(), next(it + 2));
       kblock(Index<1>(), Index<0>(), next(it + 3));
+      stretch_end(it + 2);
     }
     auto next = [&](int kb) {
       return [&, kb](int set) {
@@ -570,6 +604,11 @@ struct TileMma {
     for (; it < nk; it += 2) {
       kblock(Index<0>(), Index<1>(), next(it + 2));
       if (it + 1 < nk) kblock(Index<1>(), Index<1>(), next(it + 3));
+      stretch_end(it + 2);
+    }
+    if constexpr (STRETCHES) {
+      add(total, acc);
+      acc = total;
     }
   }
 

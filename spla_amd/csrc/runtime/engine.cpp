@@ -218,6 +218,7 @@ void enqueue_device_product(SplaOperation opA, SplaOperation opB, int64_t m, int
   if (plan.activeTiles == 0) return;  // no tile of C is needed
   d.splits = plan.splits;
   d.kSplit = plan.kSplit;
+  d.kSum = plan.kSum;
   d.tilesM = plan.tilesM;
   d.tilesN = plan.tilesN;
   d.activeTiles = plan.activeTiles;

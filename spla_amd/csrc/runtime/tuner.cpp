@@ -196,15 +196,14 @@ static GemmPlan plan_tiles(bool complex, int64_t m, int64_t n, int64_t k, int nu
         1.0, 0.5 * plan_active_tiles(m, n, rows, ts.bn / 2, fill) / static_cast<double>(tiles));
     const double needed = static_cast<double>(tiles) / allTiles;  // of C
     const int64_t kBlocks = std::max<int64_t>(1, (Kp + bk - 1) / bk);
-    const int perCU = blocks_per_cu(cfg);
-    const int64_t slots = static_cast<int64_t>(numCUs) * perCU;
     const double peak = kPeakPerCU * (8.0 / scalarBytes) * effByCfg[cfg];
     const double lone = cfg == TileL ? 0.85 : 0.88;
     // address set-up, first loads, epilogue (complex 60000 x 128 x 128: 142 us on M tiles,
     // 164 us on L tiles, which the same time for both preferred)
     const double workgroupSeconds = cfg == TileL ? 10e-6 : 2.5e-6;
     const int64_t maxSplits = std::max<int64_t>(
-        1, std::min<int64_t>(kBlocks / scalarBytes, std::max<int64_t>(64, 4 * slots / tiles)));
+        1, std::min<int64_t>(kBlocks / scalarBytes,
+                             std::max<int64_t>(64, 4 * numCUs * blocks_per_cu(cfg) / tiles)));
     int64_t lastSplits = 0;
     for (int64_t s = 1; s <= maxSplits; s += std::max<int64_t>(1, s / 32)) {
       const int64_t kb = (kBlocks + s - 1) / s;
@@ -212,10 +211,14 @@ static GemmPlan plan_tiles(bool complex, int64_t m, int64_t n, int64_t k, int nu
       if (splits == lastSplits || allTiles * splits > (int64_t(1) << 31) - 1) continue;
       lastSplits = splits;
       if (splits > 1 && splits * sums > limit) break;
-      // single precision: no longer sums than the coarse plan's, since their rounding
-      // errors grow with the length (s 4 x 10 x 309: 1.9e-7 of the result in 2 splits,
-      // 2.9e-7 in 1)
-      if (scalarBytes == 4 && kb * bk >= coarse.kSplit + bk) continue;
+      // No longer sums than the coarse plan's, since their rounding errors grow with the
+      // length (s 4 x 10 x 309: 1.9e-7 of the result in 2 splits, 2.9e-7 in 1; z 1238 x
+      // 1207 x 4119 2.6e-14 root mean square in 28 splits, 1.3e-13 in 1). Double precision
+      // has M tiles that add up sums of that length.
+      const bool longer = kb * bk >= coarse.kSplit + (scalarBytes == 4 ? bk : 1);
+      if (longer && (scalarBytes == 4 || cfg != TileM)) continue;
+      const int perCU = longer && !complex ? 3 : blocks_per_cu(cfg);  // gemm_f64_stretch_kernel
+      const int64_t slots = static_cast<int64_t>(numCUs) * perCU;
       const double work = 2.0 * ts.bm * ts.bn * bk * kb / peak;  // one workgroup on a full CU
       auto seconds = [&](int64_t groups) {
         const int64_t rounds = groups / slots, rest = groups % slots;
@@ -240,6 +243,7 @@ static GemmPlan plan_tiles(bool complex, int64_t m, int64_t n, int64_t k, int nu
         best.cfg = cfg;
         best.splits = static_cast<int>(splits);
         best.kSplit = kb * bk;
+        best.kSum = longer ? coarse.kSplit / (2 * bk) * (2 * bk) : 0;
         best.tilesM = static_cast<int>(tilesM);
         best.tilesN = static_cast<int>(tilesN);
       }

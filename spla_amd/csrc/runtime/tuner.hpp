@@ -22,6 +22,7 @@ struct GemmPlan {
   int cfg = 0;          // GemmTileConfig
   int splits = 1;       // split-K factor
   int64_t kSplit = 0;   // embedded reduction length per split
+  int64_t kSum = 0;     // embedded length of the sums a split adds up (0: one sum)
   int tilesM = 0, tilesN = 0;
   int activeTiles = 0;  // of these, the tiles that the fill mode needs
   double estSeconds = 0.0;

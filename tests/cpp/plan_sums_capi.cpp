@@ -4,7 +4,7 @@
 
 extern "C" {
 
-// out: [splits, kSplit] of the plan, [splits, kSplit] of the coarse plan, small
+// out: [splits, kSplit] of the plan, [splits, kSplit] of the coarse plan, small, kSum
 void plan_sums_c(int complex, long long m, long long n, long long k, int scalarBytes, int mode,
                  long long* out) {
   const double eff[3] = {spla_amd::Tuner::efficiency(0), spla_amd::Tuner::efficiency(1),
@@ -17,5 +17,6 @@ void plan_sums_c(int complex, long long m, long long n, long long k, int scalarB
   out[2] = c.splits;
   out[3] = c.kSplit;
   out[4] = p.small;
+  out[5] = p.kSum;
 }
 }

@@ -29,7 +29,7 @@ def plan(tmp_path_factory):
                                 ctypes.POINTER(ll)]
 
     def call(cplx, m, n, k, scalar, mode):
-        out = (ll * 5)()
+        out = (ll * 6)()
         lib.plan_sums_c(cplx, m, n, k, scalar, mode, out)
         return list(out)
 
@@ -44,6 +44,40 @@ def test_allocation_free_products_stay_accepted(plan):
     shapes += [(rng.randint(64, 9000), rng.randint(64, 9000), round(16 * 2 ** rng.uniform(0, 15)))
                for _ in range(3000)]
     for m, n, k in shapes:
-        splits, _, coarse, _, _ = plan(1, m, n, k, 8, 0)
+        splits, _, coarse, *_ = plan(1, m, n, k, 8, 0)
         if coarse == 1 or coarse * m * n * 16 <= 64 << 20:
             assert splits == 1 or splits * m * n * 16 <= 64 << 20, (m, n, k)
+
+
+@pytest.mark.parametrize("scalar", [8, 4])
+def test_sums_are_no_longer_than_the_coarse_plan(plan, scalar):
+    """The rounding error of a sum grows with its length. Small products (their own kernel) share
+    the reduction among up to 16 waves."""
+    rng = random.Random(11)
+    block = 128 // scalar
+    shapes = [(1, 1238, 1207, 4119), (1, 534, 1797, 9523), (0, 1601, 1190, 20905),
+              (1, 1560, 1626, 252100), (1, 256, 256, 4096)]
+    shapes += [(rng.randint(0, 1), *(round(2 ** rng.uniform(0, e)) for e in (12, 12, 19)))
+               for _ in range(4000)]
+    for cplx, m, n, k in shapes:
+        kp = k * (1 + cplx)
+        for mode in (0, 1, 2):
+            splits, per, coarse, longest, small, ksum = plan(cplx, m, n, k, scalar, mode)
+            if small:
+                waves = min(16, -(-k // 32))
+                step = 64 // (scalar * (1 + cplx))  # of one MFMA and 16-byte piece
+                length = -(-(-(-k // step)) // waves) * step * (1 + cplx)
+                assert length <= longest or waves == 1, (cplx, m, n, k, mode)
+                continue
+            assert ksum == 0 or (scalar == 8 and ksum % 32 == 0 and 0 < ksum < per)
+            unit = block if scalar == 4 else 1  # whole k-blocks
+            assert min(ksum or per, kp) < longest + unit, (cplx, m, n, k, mode)
+
+
+def test_shapes_that_add_up_stretches(plan):
+    """The shapes of tests/test_stretch_gpu.py take the kernel that it means to test."""
+    for cplx, m, n, k, one in [(1, 354, 550, 165, True), (1, 330, 300, 2100, False),
+                               (0, 385, 553, 301, True), (0, 400, 300, 4000, False),
+                               (1, 534, 597, 1523, False), (0, 801, 590, 3905, False)]:
+        splits, _, coarse, _, _, ksum = plan(cplx, m, n, k, 8, 0)
+        assert ksum > 0 and (splits == 1) == one and coarse > splits, (m, n, k)
