@@ -25,6 +25,8 @@ hipError_t launch_gemm_f32(const GemmDesc& d, bool complex, int layoutA, int lay
 // partial result each in d.work ([splits][n][Mp]) for launch_splitk_reduce.
 bool skinny_supported(bool complex, int layoutA, int layoutB, int64_t m, int64_t n);
 int skinny_groups(int64_t m, int64_t n);
+// Accumulators that share the sum of an output in a wave.
+int skinny_sums(bool complex, int64_t m, int64_t n);
 hipError_t launch_skinny_gemm(const GemmDesc& d, bool complex, hipStream_t stream);
 
 // Product too small for the tile kernels, in one launch (small.hip); d's tiles and

@@ -47,6 +47,12 @@ using namespace tile;
 constexpr int kWaves = 4;
 constexpr int kChunkRowBytes = 128;  // of one row and stretch
 
+// Accumulators per output: two where there are registers for them (launch bounds: 256). Real
+// m > 32 with n > 16 is the one shape with one (with two, 254 registers and 8 spilled).
+constexpr int sums_per_output(int fm, int fn, int comps, int lines) {
+  return 16 * fm * fn * comps + 6 * 2 * (fm + fn) * lines < 200 ? 2 : 1;
+}
+
 // LINES: 128-byte stretches of a row that follow each other in a chunk; ALIGNED: every
 // row starts on a cache line (see rows_aligned).
 template <bool CPLX, bool CONJ, int FM, int FN, int GROUPS, int LINES, bool ALIGNED>
@@ -64,7 +70,7 @@ __global__ void __launch_bounds__(kWaves * 64, 2) skinny_gemm_kernel(GemmDesc d)
   constexpr int kStageBytes = LINES * kLineBytes;
   constexpr int kSumBytes = FM * FN * kComps * 16 * 17 * 8;
   constexpr int kWaveBytes = kStageBytes > kSumBytes ? kStageBytes : kSumBytes;
-  constexpr int kSums = 16 * FM * FN * kComps + 6 * kLoads < 200 ? 2 : 1;  // per output
+  constexpr int kSums = sums_per_output(FM, FN, kComps, LINES);
   __shared__ __attribute__((aligned(16))) unsigned char lds[kWaves][kWaveBytes];
   typedef double loose2 __attribute__((ext_vector_type(2), aligned(8)));
 
@@ -280,6 +286,11 @@ hipError_t launch_typed(const GemmDesc& d, hipStream_t stream) {
 int skinny_groups(int64_t m, int64_t n) {
   const int64_t rows = m > n ? m : n;
   return rows > 8 ? 1 : (rows > 4 ? 2 : (rows > 2 ? 4 : (rows > 1 ? 8 : 16)));
+}
+
+int skinny_sums(bool complex, int64_t m, int64_t n) {
+  const int fm = m > 32 ? 4 : (m > 16 ? 2 : 1), fn = n > 16 ? 2 : 1;
+  return sums_per_output(fm, fn, complex ? 2 : 1, 1);
 }
 
 bool skinny_supported(bool complex, int layoutA, int layoutB, int64_t m, int64_t n) {
