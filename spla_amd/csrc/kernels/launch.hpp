@@ -20,9 +20,9 @@ hipError_t launch_gemm_f32(const GemmDesc& d, bool complex, int layoutA, int lay
                            hipStream_t stream);
 
 // Streaming FP64 / complex-FP64 product for small m, n with K-major A and B
-// (skinny.hip): the workgroups (gridDim = d.splits >= 2) take chunks of the
-// reduction in turn, 128 skinny_groups(m, n) bytes of every row each, and leave one
-// partial result each in d.work ([splits][n][Mp]) for launch_splitk_reduce.
+// (skinny.hip): the workgroups (gridDim = d.splits >= 2) take stretches of the
+// reduction in turn, one or two times 128 skinny_groups(m, n) bytes of every row, and
+// leave one partial result each in d.work ([splits][n][Mp]) for launch_splitk_reduce.
 bool skinny_supported(bool complex, int layoutA, int layoutB, int64_t m, int64_t n);
 int skinny_groups(int64_t m, int64_t n);
 // Accumulators that share the sum of an output in a wave.

@@ -53,17 +53,22 @@ constexpr int sums_per_output(int fm, int fn, int comps, int lines) {
   return 16 * fm * fn * comps + 6 * 2 * (fm + fn) * lines < 200 ? 2 : 1;
 }
 
-// LINES: 128-byte stretches of a row that follow each other in a chunk; ALIGNED: every
-// row starts on a cache line (see rows_aligned).
-template <bool CPLX, bool CONJ, int FM, int FN, int GROUPS, int LINES, bool ALIGNED>
+// LINES: 128-byte stretches of a row that follow each other in a chunk; TURN: stretches that
+// a wave takes at its turn, in TURN / LINES chunks. The turns decide which sums an element
+// goes to, so they are the same however the operands lie in memory. ALIGNED: every row
+// starts on a cache line (see rows_aligned).
+template <bool CPLX, bool CONJ, int FM, int FN, int GROUPS, int LINES, int TURN, bool ALIGNED>
 __global__ void __launch_bounds__(kWaves * 64, 2) skinny_gemm_kernel(GemmDesc d) {
   static_assert(GROUPS == 1 || (FM == 1 && FN == 1), "stretches share one fragment");
-  static_assert(GROUPS == 1 || LINES == 1, "one or the other");
+  static_assert(GROUPS == 1 || TURN == 1, "one or the other");
+  static_assert(TURN % LINES == 0, "whole chunks");
   constexpr int kComps = CPLX ? 2 : 1;
   constexpr int kElem = 8 * kComps;
   constexpr int kRows = 16 / GROUPS;  // rows of A or columns of B in a fragment
   constexpr int kChunk = kChunkRowBytes * GROUPS * LINES;  // bytes of a row in one chunk
-  constexpr int kChunkElems = kChunk / kElem;
+  constexpr int kParts = TURN / LINES;  // chunks of a turn
+  constexpr int kTurn = kChunk * kParts;
+  constexpr int kTurnElems = kTurn / kElem;
   constexpr int kPerRow = kChunk / 16;      // 16-byte pieces of a row
   constexpr int kLoadsA = 2 * FM * LINES, kLoads = 2 * (FM + FN) * LINES;  // per lane and chunk
   constexpr int kLineBytes = 16 * (FM + FN) * kRowBytes;
@@ -78,13 +83,13 @@ __global__ void __launch_bounds__(kWaves * 64, 2) skinny_gemm_kernel(GemmDesc d)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15;
   const int kk = lane >> 4;
-  // chunks of this wave: id, id + waves, id + 2 waves, ...; the partial chunk at
-  // the end of the reduction goes to the wave whose turn it is
-  const int64_t chunks = d.k / kChunkElems;
+  // turns of this wave: id, id + waves, id + 2 waves, ...; the partial one at the
+  // end of the reduction goes to the wave that is next
+  const int64_t turns = d.k / kTurnElems;
   const int64_t waves = static_cast<int64_t>(gridDim.x) * kWaves;
   const int64_t id = static_cast<int64_t>(blockIdx.x) * kWaves + wave;
-  const int64_t mine = chunks > id ? (chunks - id + waves - 1) / waves : 0;
-  const bool tail = d.k % kChunkElems != 0 && chunks % waves == id;
+  const int64_t mine = turns > id ? (turns - id + waves - 1) / waves : 0;
+  const bool tail = d.k % kTurnElems != 0 && turns % waves == id;
 
   // Piece u of a lane: row and 16-byte piece of A or B, and where it lies in LDS.
   // Rows past the operand's last one read that one: they feed outputs that are
@@ -166,7 +171,7 @@ __global__ void __launch_bounds__(kWaves * 64, 2) skinny_gemm_kernel(GemmDesc d)
   };
 
 #pragma unroll
-  for (int u = 0; u < kLoads; ++u) p[u] += id * kChunk;
+  for (int u = 0; u < kLoads; ++u) p[u] += id * kTurn;
   if (mine > 0) {
     dbl2 x[kLoads];
     auto load = [&]() {
@@ -177,28 +182,35 @@ __global__ void __launch_bounds__(kWaves * 64, 2) skinny_gemm_kernel(GemmDesc d)
       }
     };
     load();
-    const int64_t step = waves * kChunk;
-    for (int64_t c = 1; c < mine; ++c) {
+    // from the last chunk of a turn to the first of the next
+    const int64_t step = waves * kTurn - (kParts - 1) * kChunk;
+    for (int64_t c = 1; c < mine * kParts; ++c) {
+      const int64_t by = c % kParts == 0 ? step : kChunk;
 #pragma unroll
-      for (int u = 0; u < kLoads; ++u) p[u] += step;
+      for (int u = 0; u < kLoads; ++u) p[u] += by;
       compute(x, load);
     }
     compute(x, [] {});
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) p[u] += step;
   }
-  if (tail) {  // p is at the partial chunk: elements past the reduction are zero
-    const int left = static_cast<int>(d.k % kChunkElems) * kComps;  // doubles
-    dbl2 x[kLoads];
+  if (tail) {  // p is at the partial turn: elements past the reduction are zero
+    const int rest = static_cast<int>(d.k % kTurnElems) * kComps;  // doubles
 #pragma unroll
-    for (int u = 0; u < kLoads; ++u) {
-      const int at = 2 * piece_col(u);
-      const double* q = reinterpret_cast<const double*>(p[u]);
-      x[u] = dbl2{0.0, 0.0};
-      if (at < left) x[u][0] = q[0];
-      if (at + 1 < left) x[u][1] = q[1];
+    for (int part = 0; part < kParts; ++part) {
+      const int left = rest - part * (kChunk / 8);
+      if (left <= 0) break;
+      dbl2 x[kLoads];
+#pragma unroll
+      for (int u = 0; u < kLoads; ++u) {
+        const int at = 2 * piece_col(u);
+        const double* q = reinterpret_cast<const double*>(p[u] + part * kChunk);
+        x[u] = dbl2{0.0, 0.0};
+        if (at < left) x[u][0] = q[0];
+        if (at + 1 < left) x[u][1] = q[1];
+      }
+      compute(x, [] {});
     }
-    compute(x, [] {});
   }
 
   // The sums of the four waves and of the stretches, in this order, through LDS.
@@ -236,7 +248,9 @@ __global__ void __launch_bounds__(kWaves * 64, 2) skinny_gemm_kernel(GemmDesc d)
 // the caches (complex m = n = 32, k = 4000001 1013 -> 812 us; 26 x 12, 6576433 791 ->
 // 687 us), and one fragment per operand takes two stretches at a time, three lines
 // for two (m = n = 16, k = 8000001 803 -> 678 us; more fragments have no registers
-// for it).
+// for it). Rows on cache lines load one stretch at a time, the two of a turn one after the
+// other (m = n = 16, k = 8e6, whole call: complex 614 us, real 321 us; turns of one
+// stretch 635 and 335).
 bool rows_aligned(const GemmDesc& d, int elemBytes) {
   const uint64_t bits = reinterpret_cast<uintptr_t>(d.A) | reinterpret_cast<uintptr_t>(d.B) |
                         (d.m > 1 ? static_cast<uint64_t>(d.lda) * elemBytes : 0) |
@@ -248,10 +262,10 @@ template <bool CPLX, bool CONJ, int FM, int FN, int GROUPS = 1>
 hipError_t launch(const GemmDesc& d, hipStream_t stream) {
   constexpr int kLines = GROUPS == 1 && FM == 1 && FN == 1 ? 2 : 1;
   if (rows_aligned(d, CPLX ? 16 : 8))
-    hipLaunchKernelGGL((skinny_gemm_kernel<CPLX, CONJ, FM, FN, GROUPS, 1, true>), dim3(d.splits),
-                       dim3(kWaves * 64), 0, stream, d);
+    hipLaunchKernelGGL((skinny_gemm_kernel<CPLX, CONJ, FM, FN, GROUPS, 1, kLines, true>),
+                       dim3(d.splits), dim3(kWaves * 64), 0, stream, d);
   else
-    hipLaunchKernelGGL((skinny_gemm_kernel<CPLX, CONJ, FM, FN, GROUPS, kLines, false>),
+    hipLaunchKernelGGL((skinny_gemm_kernel<CPLX, CONJ, FM, FN, GROUPS, kLines, kLines, false>),
                        dim3(d.splits), dim3(kWaves * 64), 0, stream, d);
   return hipGetLastError();
 }
