@@ -54,12 +54,12 @@ template <bool CPLX, bool CONJ, int LA, int CFG, bool HALF = false, bool WIDE = 
 using BatchMma = TileMma<double, CPLX, CONJ, LA, KMajor, (CPLX ? 1 : 2) * (CFG == TileM ? 1 : 2),
                          (CFG == TileM ? 2 : 4) / (HALF ? 2 : 1), WIDE>;
 
-// One (block, tile, split) item, its tile covered by repM x repN tiles of T; on
+// One (block, tile, split) item: tile `part` of the REP x REP tiles of T that cover it; on
 // return every thread has passed the tile routine's last barrier, so the LDS
 // buffers may be reused at once.
-template <typename T, typename H, bool CPLX>
-__device__ __forceinline__ void batched_item(const BatchDesc& d, const BatchItem& it, int repM,
-                                             int repN, void* lds) {
+template <typename T, typename H, bool CPLX, int REP = 1>
+__device__ __forceinline__ void batched_item(const BatchDesc& d, const BatchItem& it, int part,
+                                             void* lds) {
   static_assert(2 * H::BN == T::BN && H::AR == T::AR, "half of the columns");
   const BatchBlock& b = d.blocks[uniform(it.block)];
   const int m = uniform(b.m), n = uniform(b.n), Mp = uniform(b.Mp), s = uniform(it.s);
@@ -86,16 +86,13 @@ __device__ __forceinline__ void batched_item(const BatchDesc& d, const BatchItem
       });
     }
   };
-#pragma unroll 1
-  for (int t = 0; t < repM * repN; ++t) {
-    const int row = (uniform(it.tm) * repM + t % repM) * T::AR;
-    const int col = (uniform(it.tn) * repN + t / repM) * T::BN;
-    if (row >= m || col >= n) continue;
-    if (n - col <= H::BN)
-      run(Type<H>(), row, col);
-    else
-      run(Type<T>(), row, col);
-  }
+  const int row = (uniform(it.tm) * REP + part % REP) * T::AR;
+  const int col = (uniform(it.tn) * REP + part / REP) * T::BN;
+  if (row >= m || col >= n) return;
+  if (n - col <= H::BN)
+    run(Type<H>(), row, col);
+  else
+    run(Type<T>(), row, col);
 }
 
 // Grouped launch: workgroup = item (gridDim.x = number of items).
@@ -104,17 +101,20 @@ __global__ void __launch_bounds__(kThreads, CFG == TileM ? 4 : 2) batched_gemm_k
   using T = BatchMma<CPLX, CONJ, LA, CFG>;
   using H = BatchMma<CPLX, CONJ, LA, CFG, true>;
   __shared__ typename T::Smem sm;
-  batched_item<T, H, CPLX>(d, d.items[blockIdx.x], 1, 1, &sm);
+  batched_item<T, H, CPLX>(d, d.items[blockIdx.x], 0, &sm);
 }
 
-// The grouped launch for blocks with wide rows (tile_wide): every tile as M tiles.
+// The grouped launch for blocks with wide rows (tile_wide): every tile as M tiles, a
+// workgroup each (BatchKernels::perItem).
+constexpr int batch_wide_rep(int cfg) { return cfg == TileM ? 1 : 2; }
+
 template <bool CPLX, bool CONJ, int LA, int CFG>
-__global__ void __launch_bounds__(kThreads, 2) batched_gemm_wide_kernel(BatchDesc d) {
+__global__ void __launch_bounds__(kThreads, 3) batched_gemm_wide_kernel(BatchDesc d) {
   using T = BatchMma<CPLX, CONJ, LA, TileM, false, true>;
   using H = BatchMma<CPLX, CONJ, LA, TileM, true, true>;
   __shared__ typename T::Smem sm;
-  constexpr int REP = CFG == TileM ? 1 : 2;
-  batched_item<T, H, CPLX>(d, d.items[blockIdx.x], REP, REP, &sm);
+  constexpr int REP = batch_wide_rep(CFG);
+  batched_item<T, H, CPLX, REP>(d, d.items[blockIdx.x / (REP * REP)], blockIdx.x % (REP * REP), &sm);
 }
 
 // Persistent launch: one workgroup per slot works through its static list of
@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(kThreads, CFG == TileM ? 4 : 2)
   __shared__ typename T::Smem sm;
   const int end = d.slotStart[blockIdx.x + 1];
   for (int i = d.slotStart[blockIdx.x]; i < end; ++i)
-    batched_item<T, H, CPLX>(d, d.items[uniform(d.slotItems[i])], 1, 1, &sm);
+    batched_item<T, H, CPLX>(d, d.items[uniform(d.slotItems[i])], 0, &sm);
 }
 
 // AR x BN: element rows and columns of a tile of the GEMM launch.
@@ -190,6 +190,7 @@ BatchKernels batched_kernels(bool complex, bool conjA, int layoutA, int cfg,
                             : reinterpret_cast<const void*>(&batched_reduce_kernel<false, 128, 128>);
   }
   k.threads = kThreads;
+  k.perItem = dispatch == BatchWide ? batch_wide_rep(cfg) * batch_wide_rep(cfg) : 1;
   return k;
 }
 

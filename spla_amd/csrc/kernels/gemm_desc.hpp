@@ -79,8 +79,10 @@ inline TileShape tile_shape(int cfg) {
 // The tile kernels address a wave's share of a tile with 32-bit lane offsets: 32
 // rows of a K-major operand or 32 reduction indices of an MN-major one. Operands
 // whose leading dimension spreads these over 4 GiB (complex doubles: from 8.1e6
-// elements) take kernels with 64-bit lane addresses, which spend vector
-// instructions on them in every k-block.
+// elements) take kernels with 64-bit lane addresses, M tiles of which a workgroup each
+// covers the planned tile (there are registers for the addresses; one or two vector
+// instructions per load): complex 64 x 64 x 8.2e6 A^H B 5.0 ms, real 100 x 100 x
+// 16.5e6 10.1 ms (with every element's address and bounds made in the loop 6.5 and 13.8).
 inline bool tile_wide(int64_t ld, int elemBytes) {
   return 33 * ld * elemBytes >= (int64_t(1) << 32);
 }

@@ -32,16 +32,17 @@ namespace {
 
 using namespace tile;
 
-// Maps the workgroup index to (split, tile row, tile column) over the active tiles of
+// Maps workgroup `bid` of G to (split, tile row, tile column) over the active tiles of
 // rows x cols. Only these are launched: workgroups that leave at once let the
 // dispatcher pile others onto their CUs (700 x 700 x 30011 complex, lower triangle, 924
 // workgroups, 3.6 per CU: 1.00 ms, with 770 empty ones among them 1.02 to 1.25 ms).
-__device__ __forceinline__ void map_block(const GemmDesc& d, int rows, int cols, int& s, int& tm,
-                                          int& tn) {
-  const int G = gridDim.x;
-  const int bid = blockIdx.x;
+// `parts` workgroups share a tile, `part` is this one's.
+__device__ __forceinline__ void map_block(const GemmDesc& d, int bid, int G, int rows, int cols,
+                                          int parts, int& s, int& tm, int& tn, int& part) {
   int lin = bid;
   if ((G & 7) == 0) lin = (bid & 7) * (G >> 3) + (bid >> 3);
+  part = lin % parts;
+  lin /= parts;
   s = lin / d.activeTiles;
   const int t = lin - s * d.activeTiles;
   if (d.fillMode != FillFull) {  // tile by tile down the columns
@@ -59,29 +60,33 @@ __device__ __forceinline__ void map_block(const GemmDesc& d, int rows, int cols,
   tn = inGroup / gsize;
 }
 
-// Body of one workgroup (shared by the FP64 and FP32 kernels): one tile of T, or
-// (MULTI) repM x repN of them one after the other. A tile of which at most half the
-// columns exist, or (not MULTI) lie in active half tiles of a fill mode, runs as the
-// half tile H: the matrix cores are what bounds the kernel, so the other half is not
+// Body of one workgroup (shared by the FP64 and FP32 kernels). A tile of the grid is one
+// of T (Whole), or repM x repN of them, one after the other (Loop) or a workgroup each
+// (Part). A tile of which at most half the columns exist, or (Whole) lie in active half
+// tiles of a fill mode, runs as the half tile H: the matrix cores are what bounds the kernel, so the other half is not
 // computed (real 100003 x 260 x 260 341 -> 326 us, a batch of 128 ragged complex blocks 14.1
 // -> 13.7 ms).
 // STRETCHES: see TileMma::run.
-template <typename T, typename H, typename S, bool CPLX, bool MULTI, bool STRETCHES = false>
+enum TileWork : int { Whole, Loop, Part };
+template <typename T, typename H, typename S, bool CPLX, TileWork WORK, bool STRETCHES = false>
 __device__ __forceinline__ void gemm_tile(const GemmDesc& d, int repM, int repN, void* lds) {
   static_assert(2 * H::BN == T::BN && H::AR == T::AR, "half of the columns");
-  if (!MULTI) repM = repN = 1;
-  int s, tm, tn;
-  map_block(d, T::AR * repM, T::BN * repN, s, tm, tn);
+  if (WORK == Whole) repM = repN = 1;
+  const int bid = WORK == Part ? blockIdx.y * gridDim.x + blockIdx.x : blockIdx.x;
+  const int G = WORK == Part ? gridDim.x * gridDim.y : gridDim.x;
+  int s, tm, tn, part;
+  map_block(d, bid, G, T::AR * repM, T::BN * repN, WORK == Part ? repM * repN : 1, s, tm, tn, part);
   s = uniform(s);
   tm = uniform(tm);
   tn = uniform(tn);
+  part = uniform(part);
   const int first = tm * T::AR * repM;
   const int col0 = tn * T::BN * repN;
   bool left = true, right = true;  // half tiles that are needed
   if (d.fillMode != FillFull) {
     const int64_t nr = min(T::AR * repM, d.m - first);
     const int64_t nc = min(T::BN * repN, d.n - col0);
-    if (!MULTI && nc > H::BN) {
+    if (WORK == Whole && nc > H::BN) {
       left = tile_active(d, first, col0, nr, H::BN);
       right = tile_active(d, first, col0 + H::BN, nr, nc - H::BN);
     }
@@ -121,11 +126,11 @@ __device__ __forceinline__ void gemm_tile(const GemmDesc& d, int repM, int repN,
     else
       run(Type<T>(), row, col);
   };
-  if constexpr (!MULTI) {
+  if constexpr (WORK == Whole) {
     one(first, col0);
   } else {
 #pragma unroll 1
-    for (int t = 0; t < repM * repN; ++t) {
+    for (int t = part; t < (WORK == Part ? part + 1 : repM * repN); ++t) {
       const int row = first + (t % repM) * T::AR, col = col0 + (t / repM) * T::BN;
       if (row < d.m && col < d.n) one(row, col);
     }
@@ -137,7 +142,7 @@ __global__ void __launch_bounds__(kThreads, MINBLOCKS) gemm_f64_kernel(GemmDesc 
   using T = TileMma<double, CPLX, CONJ, LA, LB, FM, FN>;
   using H = TileMma<double, CPLX, CONJ, LA, LB, FM, FN / 2>;
   __shared__ typename T::Smem sm;
-  gemm_tile<T, H, double, CPLX, false>(d, 1, 1, &sm);
+  gemm_tile<T, H, double, CPLX, Whole>(d, 1, 1, &sm);
 }
 
 // M tiles that add their sums up in stretches (GemmDesc::kSum), so that a product needs
@@ -151,16 +156,25 @@ __global__ void __launch_bounds__(kThreads, CPLX ? 4 : 3) gemm_f64_stretch_kerne
   using T = TileMma<double, CPLX, CONJ, LA, LB, FM, FN>;
   using H = TileMma<double, CPLX, CONJ, LA, LB, FM, FN / 2>;
   __shared__ typename T::Smem sm;
-  gemm_tile<T, H, double, CPLX, false, true>(d, 1, 1, &sm);
+  gemm_tile<T, H, double, CPLX, Whole, true>(d, 1, 1, &sm);
 }
 
 // Tiles of repM x repN of the kernel's own (see launch_layout).
-template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN, bool WIDE>
+template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN>
 __global__ void __launch_bounds__(kThreads, 2) gemm_f64_multi_kernel(GemmDesc d, int repM, int repN) {
-  using T = TileMma<double, CPLX, CONJ, LA, LB, FM, FN, WIDE>;
-  using H = TileMma<double, CPLX, CONJ, LA, LB, FM, FN / 2, WIDE>;
+  using T = TileMma<double, CPLX, CONJ, LA, LB, FM, FN>;
+  using H = TileMma<double, CPLX, CONJ, LA, LB, FM, FN / 2>;
   __shared__ typename T::Smem sm;
-  gemm_tile<T, H, double, CPLX, true, WIDE>(d, repM, repN, &sm);
+  gemm_tile<T, H, double, CPLX, Loop>(d, repM, repN, &sm);
+}
+
+// The same with a workgroup for each of them, operands with wide rows (tile_wide).
+template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN>
+__global__ void __launch_bounds__(kThreads, 3) gemm_f64_wide_kernel(GemmDesc d, int repM, int repN) {
+  using T = TileMma<double, CPLX, CONJ, LA, LB, FM, FN, true>;
+  using H = TileMma<double, CPLX, CONJ, LA, LB, FM, FN / 2, true>;
+  __shared__ typename T::Smem sm;
+  gemm_tile<T, H, double, CPLX, Part, true>(d, repM, repN, &sm);
 }
 
 template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN, int MINBLOCKS>
@@ -168,16 +182,25 @@ __global__ void __launch_bounds__(kThreads, MINBLOCKS) gemm_f32_kernel(GemmDesc 
   using T = TileMma<float, CPLX, CONJ, LA, LB, FM, FN>;
   using H = TileMma<float, CPLX, CONJ, LA, LB, FM, FN / 2>;
   __shared__ typename T::Smem sm;
-  gemm_tile<T, H, float, CPLX, false>(d, 1, 1, &sm);
+  gemm_tile<T, H, float, CPLX, Whole>(d, 1, 1, &sm);
 }
 
 // Tiles of repM x repN of the kernel's own (see launch_layout).
-template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN, bool WIDE>
+template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN>
 __global__ void __launch_bounds__(kThreads, 2) gemm_f32_multi_kernel(GemmDesc d, int repM, int repN) {
-  using T = TileMma<float, CPLX, CONJ, LA, LB, FM, FN, WIDE>;
-  using H = TileMma<float, CPLX, CONJ, LA, LB, FM, FN / 2, WIDE>;
+  using T = TileMma<float, CPLX, CONJ, LA, LB, FM, FN>;
+  using H = TileMma<float, CPLX, CONJ, LA, LB, FM, FN / 2>;
   __shared__ typename T::Smem sm;
-  gemm_tile<T, H, float, CPLX, true>(d, repM, repN, &sm);
+  gemm_tile<T, H, float, CPLX, Loop>(d, repM, repN, &sm);
+}
+
+// The same with a workgroup for each of them, operands with wide rows (tile_wide).
+template <bool CPLX, bool CONJ, int LA, int LB, int FM, int FN>
+__global__ void __launch_bounds__(kThreads, 3) gemm_f32_wide_kernel(GemmDesc d, int repM, int repN) {
+  using T = TileMma<float, CPLX, CONJ, LA, LB, FM, FN, true>;
+  using H = TileMma<float, CPLX, CONJ, LA, LB, FM, FN / 2, true>;
+  __shared__ typename T::Smem sm;
+  gemm_tile<T, H, float, CPLX, Part>(d, repM, repN, &sm);
 }
 
 // Adds the split-K partial sums in split order and applies alpha / beta.
@@ -295,12 +318,14 @@ hipError_t launch_layout(const GemmDesc& d, int cfg, hipStream_t stream) {
   const int elem = (F32 ? 4 : 8) * (CPLX ? 2 : 1);
   if (tile_wide(d.lda, elem) || tile_wide(d.ldb, elem)) {
     const TileShape ts = tile_shape(cfg), tm = tile_shape(TileM);
+    const int repM = ts.bm / tm.bm, repN = ts.bn / tm.bn;
+    const dim3 wide(grid.x, repM * repN);  // two counts: threads along x fit 32 bits
     if constexpr (F32)
-      hipLaunchKernelGGL((gemm_f32_multi_kernel<CPLX, CONJ, LA, LB, R, 2, true>), grid, block, 0,
-                         stream, d, ts.bm / tm.bm, ts.bn / tm.bn);
+      hipLaunchKernelGGL((gemm_f32_wide_kernel<CPLX, CONJ, LA, LB, R, 2>), wide, block, 0, stream,
+                         d, repM, repN);
     else
-      hipLaunchKernelGGL((gemm_f64_multi_kernel<CPLX, CONJ, LA, LB, R, 2, true>), grid, block, 0,
-                         stream, d, ts.bm / tm.bm, ts.bn / tm.bn);
+      hipLaunchKernelGGL((gemm_f64_wide_kernel<CPLX, CONJ, LA, LB, R, 2>), wide, block, 0, stream,
+                         d, repM, repN);
     return hipGetLastError();
   }
   if constexpr (F32) {
@@ -310,7 +335,7 @@ hipError_t launch_layout(const GemmDesc& d, int cfg, hipStream_t stream) {
                            d);
         break;
       case TileXL:
-        hipLaunchKernelGGL((gemm_f32_multi_kernel<CPLX, CONJ, LA, LB, 2 * R, 4, false>), grid,
+        hipLaunchKernelGGL((gemm_f32_multi_kernel<CPLX, CONJ, LA, LB, 2 * R, 4>), grid,
                            block, 0, stream, d, 2, 1);
         break;
       default:
@@ -329,7 +354,7 @@ hipError_t launch_layout(const GemmDesc& d, int cfg, hipStream_t stream) {
                              stream, d);
         break;
       case TileXL:
-        hipLaunchKernelGGL((gemm_f64_multi_kernel<CPLX, CONJ, LA, LB, 2 * R, 4, false>), grid,
+        hipLaunchKernelGGL((gemm_f64_multi_kernel<CPLX, CONJ, LA, LB, 2 * R, 4>), grid,
                            block, 0, stream, d, 2, 1);
         break;
       default:

@@ -58,13 +58,14 @@ hipError_t launch_crt(bool complex, const CrtDesc& d, int limbs, hipStream_t str
 // a tile configuration (TileL or TileM) and A layout (KMajor: ssb blocks, conjA for
 // A^H; MNMajor: sbs blocks), as kernel handles for hipLaunchKernel and
 // hipGraphAddKernelNode; `threads` per workgroup. Dispatch of the GEMM kernel: one
-// workgroup per BatchItem, the same for blocks with wide rows (tile_wide), or one
+// workgroup per BatchItem, `perItem` of them for blocks with wide rows (tile_wide), or one
 // workgroup per slot of the static schedule.
 enum BatchDispatch : int { BatchGrouped = 0, BatchWide = 1, BatchPersistent = 2 };
 struct BatchKernels {
   const void* gemm;
   const void* reduce;
   int threads;
+  int perItem;  // workgroups of the GEMM kernel to an item
 };
 BatchKernels batched_kernels(bool complex, bool conjA, int layoutA, int cfg,
                              BatchDispatch dispatch);

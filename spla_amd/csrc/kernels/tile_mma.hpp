@@ -150,8 +150,9 @@ struct TileOperands {
 // Moves ROWS rows x one k-block of an operand from global memory through
 // registers to LDS.
 // WIDE: rows (K-major) or reduction indices (MN-major) so far apart that 32-bit
-// lane offsets do not reach over a wave's pieces (tile_wide of gemm_desc.hpp); 64-bit lane
-// addresses, made for every k-block.
+// lane offsets do not reach over a wave's pieces (tile_wide of gemm_desc.hpp): 64-bit lane
+// addresses, one per piece (K-major) or one of the first (MN-major), to which a wave-uniform
+// distance is added for every load.
 template <typename S, bool CPLX, int LAYOUT, int ROWS, bool WIDE>
 struct TileStage {
   static constexpr int kComps = CPLX ? 2 : 1;
@@ -177,12 +178,13 @@ struct TileStage {
   static constexpr int kWaveRows = ROWS / 4;
   static constexpr int kOffs = LAYOUT == KMajor ? kPieces : 1;
   const char* origin;   // the tile's first row, first reduction index
-  const char* base;     // the wave's first row or reduction index
+  const char* base;     // the wave's first row or reduction index (WIDE: the tile's)
   int last;             // last row that exists, relative to the tile
   int64_t rowBytes;
   int64_t blockStep;    // bytes from one k-block to the next
   uint32_t pieceStep;
   uint32_t off[kOffs];
+  const char* address[WIDE ? kOffs : 1];  // WIDE: in place of the offsets
   int64_t kEnd;         // reduction range in elements, relative to k-block 0
   int fast;             // k-blocks 0 .. fast - 1 are whole
 
@@ -190,12 +192,6 @@ struct TileStage {
   __device__ __forceinline__ static int tile_row(int tid, int u) {
     return LAYOUT == KMajor ? (tid >> 6) * kWaveRows + 8 * u + ((tid & 63) >> 3) : tid % ROWS;
   }
-  // Reduction index (relative to k-block 0) of the first element of piece u of k-block kb.
-  __device__ __forceinline__ static int64_t first_index(int tid, int u, int kb) {
-    return static_cast<int64_t>(kb) * kBK +
-           (LAYOUT == KMajor ? kPerChunk * (tid & 7) : (tid + kThreads * u) / ROWS);
-  }
-
   // rows [rowBase, limit) of the operand at X exist (at least one); reduction
   // elements [k0, k1).
   __device__ __forceinline__ void init(const S* X, int64_t ld, int rowBase, int limit, int64_t k0,
@@ -210,7 +206,18 @@ struct TileStage {
     kEnd = k1 - k0;
     rowBytes = LAYOUT == KMajor ? ldBytes : kElem;
     origin = x + k0 * (LAYOUT == KMajor ? kElem : ldBytes);
-    if (LAYOUT == KMajor) {
+    fast = static_cast<int>(kEnd / kBK);
+    if constexpr (WIDE) {
+      base = origin;
+      blockStep = LAYOUT == KMajor ? kBlockBytes : kBK * ldBytes;
+#pragma unroll
+      for (int u = 0; u < kOffs; ++u) {
+        const int64_t row = min(tile_row(threadIdx.x, u), last);
+        address[u] = LAYOUT == KMajor
+                         ? origin + row * ldBytes + kChunk * (lane & 7)
+                         : origin + (threadIdx.x / ROWS) * ldBytes + row * kElem;
+      }
+    } else if (LAYOUT == KMajor) {
       const int first = min(wave * kWaveRows, last);
       base = origin + first * ldBytes;
       blockStep = kBlockBytes;
@@ -228,7 +235,6 @@ struct TileStage {
       off[0] = static_cast<uint32_t>(min(tile_row(threadIdx.x, 0), last)) * kElem;
       if (ROWS < 64) off[0] += static_cast<uint32_t>(lane / ROWS) * ld32;
     }
-    fast = WIDE ? 0 : static_cast<int>(kEnd / kBK);
   }
 
   // readfirstlane: wave-uniform already, but kept in scalar registers for certain
@@ -243,6 +249,15 @@ struct TileStage {
   // k-block kb < fast. Buffer loads: the base is four scalar registers, the lane
   // offset one vector register that never changes.
   __device__ __forceinline__ void load_fast(Regs& r, int kb) const {
+    if constexpr (WIDE) {
+      using Loose = typename VecOf<S, kScalars>::loose;
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u)
+        r.p[u] = *reinterpret_cast<const Loose*>(
+            LAYOUT == KMajor ? address[u] + kb * blockStep
+                             : address[0] + (kb * kBK + u * (kThreads / ROWS)) * (blockStep / kBK));
+      return;
+    }
     const __amdgpu_buffer_rsrc_t rsrc = resource(base + kb * blockStep);
 #pragma unroll
     for (int u = 0; u < kPieces; ++u)
@@ -255,7 +270,7 @@ struct TileStage {
   // operands; they are read from the range's last element, so that every load is
   // issued without a branch. A k-block past the range leaves r as it is.
   __device__ __forceinline__ void load(Regs& r, int kb) const {
-    if (!WIDE && kb < fast) return load_fast(r, kb);
+    if (kb < fast) return load_fast(r, kb);
     const int64_t left = kEnd - static_cast<int64_t>(kb) * kBK;
     if (left <= 0) return;
     const int rem = static_cast<int>(min(left, static_cast<int64_t>(kBK)));

@@ -202,10 +202,11 @@ void GroupedLaunch::build(spla::ContextInternal& ctx, bool complex, SplaOperatio
   kernels_ = batched_kernels(complex, desc_.conjA != 0, opA == SPLA_OP_NONE ? MNMajor : KMajor,
                              sched.cfg,
                              wide ? BatchWide : persistent ? BatchPersistent : BatchGrouped);
-  // GEMM workgroups: one per item (grouped) or one per slot (persistent)
-  numItems_ = sched.items.empty() ? 0u
-                                  : static_cast<unsigned>(persistent ? sched.slotStart.size() - 1
-                                                                     : sched.items.size());
+  // GEMM workgroups: per item (grouped, wide) or one per slot (persistent)
+  numItems_ = sched.items.empty()
+                  ? 0u
+                  : static_cast<unsigned>(persistent ? sched.slotStart.size() - 1
+                                                     : sched.items.size() * kernels_.perItem);
   numReduce_ = static_cast<unsigned>(sched.reduce.size());
   persistent_ = persistent;
   if (withGraph && numItems_ > 0) {
