@@ -117,6 +117,20 @@ __global__ void __launch_bounds__(kThreads, 3) batched_gemm_wide_kernel(BatchDes
   batched_item<T, H, CPLX, REP>(d, d.items[blockIdx.x / (REP * REP)], blockIdx.x % (REP * REP), &sm);
 }
 
+// The persistent launch for blocks with wide rows.
+template <bool CPLX, bool CONJ, int LA, int CFG>
+__global__ void __launch_bounds__(kThreads, 3) batched_gemm_wide_persistent_kernel(BatchDesc d) {
+  using T = BatchMma<CPLX, CONJ, LA, TileM, false, true>;
+  using H = BatchMma<CPLX, CONJ, LA, TileM, true, true>;
+  __shared__ typename T::Smem sm;
+  constexpr int REP = batch_wide_rep(CFG);
+  const int end = d.slotStart[blockIdx.x + 1];
+  for (int i = d.slotStart[blockIdx.x]; i < end; ++i)
+#pragma unroll 1
+    for (int part = 0; part < REP * REP; ++part)
+      batched_item<T, H, CPLX, REP>(d, d.items[uniform(d.slotItems[i])], part, &sm);
+}
+
 // Persistent launch: one workgroup per slot works through its static list of
 // items (gridDim.x = number of slots); no workgroup waits for another.
 template <bool CPLX, bool CONJ, int LA, int CFG>
@@ -161,6 +175,9 @@ const void* gemm_kernel_of(BatchDispatch dispatch) {
       return reinterpret_cast<const void*>(&batched_gemm_persistent_kernel<CPLX, CONJ, LA, CFG>);
     case BatchWide:
       return reinterpret_cast<const void*>(&batched_gemm_wide_kernel<CPLX, CONJ, LA, CFG>);
+    case BatchWidePersistent:
+      return reinterpret_cast<const void*>(
+          &batched_gemm_wide_persistent_kernel<CPLX, CONJ, LA, CFG>);
     default:
       return reinterpret_cast<const void*>(&batched_gemm_kernel<CPLX, CONJ, LA, CFG>);
   }

@@ -59,8 +59,13 @@ hipError_t launch_crt(bool complex, const CrtDesc& d, int limbs, hipStream_t str
 // A^H; MNMajor: sbs blocks), as kernel handles for hipLaunchKernel and
 // hipGraphAddKernelNode; `threads` per workgroup. Dispatch of the GEMM kernel: one
 // workgroup per BatchItem, `perItem` of them for blocks with wide rows (tile_wide), or one
-// workgroup per slot of the static schedule.
-enum BatchDispatch : int { BatchGrouped = 0, BatchWide = 1, BatchPersistent = 2 };
+// workgroup per slot of the static schedule, with a kernel for wide rows as well.
+enum BatchDispatch : int {
+  BatchGrouped = 0,
+  BatchWide = 1,
+  BatchPersistent = 2,
+  BatchWidePersistent = 3
+};
 struct BatchKernels {
   const void* gemm;
   const void* reduce;

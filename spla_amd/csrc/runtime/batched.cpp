@@ -47,6 +47,14 @@ bool on_device(const void* p) {
   return attr.type == hipMemoryTypeDevice;
 }
 
+// Whether the launch needs the kernels for wide rows (one such block is enough).
+bool wide_rows(const std::vector<BlockSpec>& specs, bool complex) {
+  const int elem = complex ? 16 : 8;
+  return std::any_of(specs.begin(), specs.end(), [elem](const BlockSpec& b) {
+    return tile_wide(b.lda, elem) || tile_wide(b.ldb, elem);
+  });
+}
+
 // Split-precision batch in three rounds over the lanes: the statistics of
 // every block, one synchronization and the host plans of all blocks, then the
 // residue planes, INT8 GEMMs and reconstructions (blocks that fall back run
@@ -195,13 +203,11 @@ void GroupedLaunch::build(spla::ContextInternal& ctx, bool complex, SplaOperatio
   desc_.betaZero = (desc_.betaRe == 0.0 && desc_.betaIm == 0.0) ? 1 : 0;
   desc_.conjA = (complex && opA == SPLA_OP_CONJ_TRANSPOSE) ? 1 : 0;
   desc_.conjB = 0;
-  bool wide = false;
-  for (const BlockSpec& sp : specs)
-    wide |= tile_wide(sp.lda, complex ? 16 : 8) || tile_wide(sp.ldb, complex ? 16 : 8);
-  if (wide) persistent = false;
+  const BatchDispatch dispatch =
+      wide_rows(specs, complex) ? (persistent ? BatchWidePersistent : BatchWide)
+                                : (persistent ? BatchPersistent : BatchGrouped);
   kernels_ = batched_kernels(complex, desc_.conjA != 0, opA == SPLA_OP_NONE ? MNMajor : KMajor,
-                             sched.cfg,
-                             wide ? BatchWide : persistent ? BatchPersistent : BatchGrouped);
+                             sched.cfg, dispatch);
   // GEMM workgroups: per item (grouped, wide) or one per slot (persistent)
   numItems_ = sched.items.empty()
                   ? 0u
@@ -304,9 +310,11 @@ BatchPlan::BatchPlan(std::shared_ptr<spla::ContextInternal> ctx, bool complex, S
         }
       }
     measuredMs_ = bestMs;
-    const double eff = ctx_->batch_efficiency(best.cfg) * best.modelSeconds / (bestMs * 1e-3);
-    ctx_->set_batch_efficiency(best.cfg, std::min(0.95, std::max(0.05, eff)));
-    ctx_->set_batch_persistent(persistent);
+    if (!wide_rows(specs_, complex_)) {  // else measured on kernels that few batches run
+      const double eff = ctx_->batch_efficiency(best.cfg) * best.modelSeconds / (bestMs * 1e-3);
+      ctx_->set_batch_efficiency(best.cfg, std::min(0.95, std::max(0.05, eff)));
+      ctx_->set_batch_persistent(persistent);
+    }
   }
   sched_ = std::move(best);
   full_.build(*ctx_, complex_, opA_, specs_, alpha_, beta_, sched_, persistent,

@@ -70,7 +70,8 @@ def test_stretches(ctx, device, dtype, m, n, k):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.complex128], ids=["d", "z"])
 @pytest.mark.parametrize("opA", "CN")
-def test_batches(ctx, device, dtype, opA):
+@pytest.mark.parametrize("persistent", [False, True], ids=["grouped", "persistent"])
+def test_batches(ctx, device, dtype, opA, persistent):
     """Blocks of one to several tiles and k-blocks beside one with wide rows, more than enough of
     them for large tiles as well."""
     opA = "T" if opA == "C" and dtype == np.float64 else opA
@@ -86,10 +87,36 @@ def test_batches(ctx, device, dtype, opA):
         keep.append((dA, dB, dC))
         specs.append(dict(m=m, n=n, k=k, A=dA, lda=lda, B=dB, ldb=k, C=dC, ldc=m))
         want.append(apply(opA, to_matrix(A, ra, ca, ra)) @ to_matrix(B, k, n, k))
-    with_batch = spla.Batch(ctx, specs, 1.0, 0.0, complex_=dtype == np.complex128, opA=OPS[opA])
-    with_batch.execute()
+    batch = spla.Batch(ctx, specs, 1.0, 0.0, complex_=dtype == np.complex128, opA=OPS[opA],
+                       persistent=persistent)
+    assert batch.info()["persistent"] == persistent
+    batch.execute()
     for (m, n, k), (_, _, dC), ref in zip(sizes, keep, want):
         assert np.array_equal(to_matrix(dC.cpu().numpy(), m, n, m), ref), (m, n, k)
-    with_batch.close()
+    batch.close()
     del keep, specs
     torch.cuda.empty_cache()
+
+
+def test_measuring_leaves_the_context_alone(device):
+    """A batch with wide rows that measures its candidates does not decide how the context runs
+    ordinary batches: their plans are the same as without it."""
+    def ordinary(ctx):
+        x = torch.zeros(500 * 300, dtype=torch.float64, device=device)
+        c = torch.zeros(300 * 300, dtype=torch.float64, device=device)
+        specs = [dict(m=300, n=290 - i, k=500, A=x, lda=500, B=x, ldb=500, C=c, ldc=300)
+                 for i in range(40)]
+        batch = spla.Batch(ctx, specs, 1.0, 0.0, complex_=False, opA=OPS["T"])
+        info = batch.info()
+        batch.close()
+        return info
+
+    contexts = [spla.Context(spla.ProcessingUnit.GPU) for _ in range(2)]
+    ld = wide_ld(np.float64)
+    x = torch.zeros(ld * 15 + 400, dtype=torch.float64, device=device)
+    c = torch.zeros(256, dtype=torch.float64, device=device)
+    specs = [dict(m=16, n=16, k=400, A=x, lda=ld, B=x, ldb=400, C=c, ldc=16)]
+    measured = spla.Batch(contexts[1], specs, 1.0, 0.0, complex_=False, opA=OPS["T"],
+                          measure=True)
+    measured.close()
+    assert ordinary(contexts[0]) == ordinary(contexts[1])
