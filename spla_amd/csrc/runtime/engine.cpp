@@ -144,6 +144,8 @@ static_assert(kSkinnyMinKp * 8 >= 2 * 16 * kSkinnyChunkBytes * kSkinnyChunksPerW
 
 // `fixed` (optional): caller-provided split-K workspace; nothing is allocated,
 // and a plan whose partial sums exceed it raises GPUAllocationError.
+// `tiles` (optional): plan of a reduction at least as long, whose tiles and length of a
+// split are taken.
 struct FixedWorkspace {
   void* ptr;
   std::size_t bytes;
@@ -155,7 +157,8 @@ void enqueue_device_product(SplaOperation opA, SplaOperation opB, int64_t m, int
                             T* C, int64_t ldc, spla::ContextInternal& ctx, const FillSpec& fill,
                             hipStream_t stream, std::vector<Block>& keep, Block* reuse = nullptr,
                             bool trySplit = true, bool wholeChip = true,
-                            const FixedWorkspace* fixed = nullptr) {
+                            const FixedWorkspace* fixed = nullptr,
+                            const GemmPlan* tiles = nullptr) {
   using S = Scalar<T>;
   constexpr bool cplx = S::kComplex;
   constexpr bool f32 = S::kF32;
@@ -196,10 +199,16 @@ void enqueue_device_product(SplaOperation opA, SplaOperation opB, int64_t m, int
   GemmPlan plan =
       ctx.tuner().plan(cplx, la, lb, m, n, k, ctx.num_cus(), wholeChip, f32 ? 4 : 8,
                        PlanFill{d.fillMode, d.fillRowOff, d.fillColOff});
+  if (tiles) {
+    const double seconds = plan.estSeconds;
+    plan = *tiles;
+    plan.estSeconds = seconds;
+    plan.splits = static_cast<int>((d.Kp + plan.kSplit - 1) / plan.kSplit);
+  }
   // Small m, n with a long reduction on a whole device: HBM-bound, streamed by
-  // the skinny kernel (one workgroup per split, no LDS staging).
+  // the skinny kernel (the workgroups take stretches of the reduction in turn).
   // (at kSkinnyMinKp two workgroups have their chunks: always several splits)
-  const bool skinny = !f32 && wholeChip && skinny_supported(cplx, la, lb, m, n) &&
+  const bool skinny = !f32 && wholeChip && !tiles && skinny_supported(cplx, la, lb, m, n) &&
                       d.Kp >= kSkinnyMinKp;
   if (skinny) {
     const int64_t chunks = d.Kp * 8 / (kSkinnyChunkBytes * skinny_groups(m, n));
@@ -386,6 +395,16 @@ void gemm_gpu_f64(SplaOperation opA, SplaOperation opB, int64_t m, int64_t n, in
     }
     Event copied[kSlots], computed[kSlots];
     Block workspace;
+    // A fill mode's chunks add up on the same tiles: else an element beside the triangle
+    // gets the sum of some of them.
+    GemmPlan tiles;
+    const bool sameTiles = fill.mode != SPLA_FILL_MODE_FULL && numChunks > 1;
+    if (sameTiles) {
+      tiles = ctx.tuner().plan(Scalar<T>::kComplex, kMajorA ? KMajor : MNMajor,
+                               kMajorB ? KMajor : MNMajor, m, n, kc, ctx.num_cus(), true, 8,
+                               PlanFill{fill.mode, fill.rowOff, fill.colOff});
+      tiles.small = false;
+    }
 
     auto stage = [&](const T* X, int64_t ldx, bool kMajor, int64_t outer, MemKind kind,
                      Block& dev, Block& pin, int64_t k0, int64_t kcur, int slot) {
@@ -429,7 +448,8 @@ void gemm_gpu_f64(SplaOperation opA, SplaOperation opB, int64_t m, int64_t n, in
       // SPLA multiply_gpu applies beta to the first chunk only (multiply_gpu.cpp:141).
       const T betaChunk = (c == 0) ? beta : T(1);
       enqueue_device_product(opA, opB, m, n, kcur, alpha, cA, cLda, cB, cLdb, betaChunk, dC, dldc,
-                             ctx, fill, stream, keep, &workspace);
+                             ctx, fill, stream, keep, &workspace, /*trySplit=*/true,
+                             /*wholeChip=*/true, nullptr, sameTiles ? &tiles : nullptr);
       hip_check(hipEventRecord(computed[slot].get(), stream));
     }
   }
