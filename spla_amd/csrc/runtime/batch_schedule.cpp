@@ -14,6 +14,12 @@ constexpr double kPeakPerCU = 128.0 * 2.4e9;  // FP64 matrix flop / s per CU
 constexpr double kItemOverhead = 2.0e-6;      // prologue + epilogue per workgroup
 constexpr double kLaunchOverhead = 8.0e-6;    // per launch in the graph
 constexpr double kReduceBytesPerSecond = 4.0e12;
+// A thread of the reduction adds the partial sums of its elements one after the other, with
+// eight loads in flight (20 real blocks up to 512 x 512 x 65536 on small tiles: 0.49, 0.53,
+// 0.62 and 0.74 ms with up to 64, 128, 256 and 256 splits, of which the products take 0.3
+// ms; 0.68, 0.94, 1.45 and 1.90 ms with one load after the other).
+constexpr double kReduceLoadSeconds = 0.07e-6;
+constexpr int kReduceThreads = 256;
 constexpr int kMinKBlocksPerSplit = 16;
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -82,7 +88,7 @@ BatchSchedule plan_batch_schedule(const std::vector<BatchShape>& shapes, bool co
     if (s.m <= 0 || s.n <= 0) continue;
     const int64_t Kp = alphaZero ? 0 : s.k * comps;
     const int64_t kBlocks = ceil_div(Kp, ts.bk);
-    int64_t sp = static_cast<int64_t>(std::ceil(tileCost[b] * splitScale / target));
+    int64_t sp = static_cast<int64_t>(std::ceil(tileCost[b] * splitScale / target - 1e-6));
     sp = std::max<int64_t>(1, std::min<int64_t>(sp, std::max<int64_t>(1, kBlocks /
                                                                        kMinKBlocksPerSplit)));
     const int64_t kbPer = kBlocks > 0 ? ceil_div(kBlocks, sp) : 1;
@@ -108,6 +114,7 @@ BatchSchedule plan_batch_schedule(const std::vector<BatchShape>& shapes, bool co
   std::vector<std::pair<double, int>> order(tiles.size());  // (cost of a split, tile)
   std::size_t count = 0;
   double reduceSeconds = 0.0;
+  int mostSplits = 0;
   for (std::size_t i = 0; i < tiles.size(); ++i) {
     const Tile& t = tiles[i];
     const BatchBlock& bb = out.blocks[t.block];
@@ -115,6 +122,7 @@ BatchSchedule plan_batch_schedule(const std::vector<BatchShape>& shapes, bool co
     count += bb.splits;
     if (bb.splits > 1) {
       out.reduce.push_back({t.block, t.tm, t.tn});
+      mostSplits = std::max(mostSplits, bb.splits);
       reduceSeconds +=
           (bb.splits + 2.0) * ar * ts.bn * 8.0 * comps / kReduceBytesPerSecond;
     }
@@ -159,6 +167,8 @@ BatchSchedule plan_batch_schedule(const std::vector<BatchShape>& shapes, bool co
   std::vector<int> next(out.slotStart.begin(), out.slotStart.end() - 1);
   for (std::size_t i = 0; i < items.size(); ++i)
     out.slotItems[next[slotOf[i]]++] = static_cast<int>(i);
+  reduceSeconds = std::max(reduceSeconds, static_cast<double>(mostSplits) *
+                                              (ar * ts.bn / kReduceThreads) * kReduceLoadSeconds);
   out.modelSeconds = makespan + reduceSeconds + kLaunchOverhead * (out.reduce.empty() ? 1 : 2);
   return out;
 }

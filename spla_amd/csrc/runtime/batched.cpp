@@ -335,10 +335,7 @@ BatchSchedule BatchPlan::schedule(const std::vector<BlockSpec>& specs, int cfg,
 }
 
 BatchSchedule BatchPlan::best_schedule(const std::vector<BlockSpec>& specs) const {
-  // Half as long splits on the small tiles: 128 ragged complex blocks 13.2 -> 12.8 ms,
-  // and the model, which gives a lone workgroup a quarter of its CU, comes close enough
-  // to choose these tiles (20 such blocks: 2.28 ms, 2.97 ms on large tiles, which it
-  // preferred).
+  // Half as long splits on the small tiles, as long as those on the large ones.
   BatchSchedule best = schedule(specs, TileL, 1.0);
   BatchSchedule other = schedule(specs, TileM, 2.0);
   if (other.modelSeconds < best.modelSeconds) std::swap(best, other);
@@ -390,7 +387,11 @@ void BatchPlan::execute() {
   // block's own FP64 estimate) stay on FP64; the others are split candidates.
   // The candidates would otherwise join the grouped launch, so they run split
   // only when their lower bounds, one after another on the whole chip, beat
-  // the grouped launch's model time for them.
+  // kSplitMargin of the grouped launch's model time for them: split batches take 1.35 to
+  // 1.45 times their lower bound, the grouped launch 1.0 to 1.1 times its model (8 blocks up
+  // to 1024 x 1024 x 65536: complex 22.8 and 27.5 ms, bound 0.55 of the model; real 8.3 and
+  // 8.0 ms, 0.9 of it).
+  constexpr double kSplitMargin = 0.75;
   std::vector<BlockSpec> fp64, split;
   std::vector<char> mask;
   bool allFp64 = mode == GemmModeFP64 || alphaZero;
@@ -405,7 +406,7 @@ void BatchPlan::execute() {
       if (mask[i]) splitSeconds += lower;
       (mask[i] ? split : fp64).push_back(b);
     }
-    allFp64 = split.empty() || splitSeconds >= 0.95 * best_schedule(split).modelSeconds;
+    allFp64 = split.empty() || splitSeconds >= kSplitMargin * best_schedule(split).modelSeconds;
   }
   if (allFp64) {
     // the grouped GEMM and the split reduction, replayed from the graph

@@ -115,8 +115,9 @@ private:
   std::size_t deviceMemory_ = 0;
 
   spla_amd::Tuner tuner_;
-  // TileL, TileM: over the model's time, 0.76 and 0.85 to 0.91 on ragged complex blocks
-  double batchEfficiency_[2] = {0.85, 0.88};
+  // TileL, TileM: what batches of 8 to 512 blocks ran at by the model's count, 0.86 to 0.98
+  // and 0.73 to 0.89; with these two the model took the faster shape for all of 13 batches
+  double batchEfficiency_[2] = {0.93, 0.83};
   bool batchPersistent_ = false;
   int gemmMode_ = 0;
   double splitTolerance_ = 1e-14;
