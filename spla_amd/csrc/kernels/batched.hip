@@ -54,7 +54,7 @@ template <bool CPLX, bool CONJ, int LA, int CFG, bool HALF = false, bool WIDE = 
 using BatchMma = TileMma<double, CPLX, CONJ, LA, KMajor, (CPLX ? 1 : 2) * (CFG == TileM ? 1 : 2),
                          (CFG == TileM ? 2 : 4) / (HALF ? 2 : 1), WIDE>;
 
-// One (block, tile, split) item: tile `part` of the REP x REP tiles of T that cover it; on
+// One (block, tile, split) item, or tile `part` of the REP x REP tiles of T that cover it; on
 // return every thread has passed the tile routine's last barrier, so the LDS
 // buffers may be reused at once.
 template <typename T, typename H, bool CPLX, int REP = 1>

@@ -6,8 +6,9 @@
 // complex product is four real products per pair of elements, exactly 8*m*n*k
 // flops, with no operand expanded in memory. Its sizes are given as those of
 // one real GEMM of size (2m) x n x (2k), the "embedded" sizes Mp and Kp:
-// q = 2*l + c runs over the real (c = 0) and imaginary (c = 1) parts. Split-K partial sums are stored as interleaved
-// (re, im) pairs, i.e. in C's own column-major complex layout.
+// q = 2*l + c runs over the real (c = 0) and imaginary (c = 1) parts. Split-K partial
+// sums are stored as interleaved (re, im) pairs, i.e. in C's own column-major complex
+// layout.
 #pragma once
 
 #include <cstdint>
@@ -56,8 +57,8 @@ struct GemmDesc {
 // Tile configurations of the FP64 MFMA kernel. Rows are embedded rows.
 enum GemmTileConfig : int {
   TileL = 0,   // 128 x 128 block, 4 waves of 64 x 64, 2 blocks per CU
-  TileM = 1,   // 64 x 64 block, 4 waves of 32 x 32
-  TileXL = 2,  // 256 x 128 block, 4 waves of 128 x 64, 1 block per CU
+  TileM = 1,   // 64 x 64 block, 4 waves of 32 x 32, 4 blocks per CU
+  TileXL = 2,  // 256 x 128 block: two L tiles in turn, 2 blocks per CU (opt-in)
   NumTileConfigs = 3
 };
 

@@ -309,7 +309,7 @@ __global__ void __launch_bounds__(256) scale_kernel(GemmDesc d) {
 // Wave tiles: L 64 x 64 embedded rows and columns (two workgroups per CU), M
 // 32 x 32 (four); XL is two L tiles one after the other (128 x 64 wave tiles, one
 // wave per SIMD, keep the compiler moving accumulators between register files).
-// Operands with wide rows (tile_wide) run every shape as M tiles.
+// Operands with wide rows (tile_wide) run every shape as M tiles, a workgroup each.
 template <bool F32, bool CPLX, bool CONJ, int LA, int LB>
 hipError_t launch_layout(const GemmDesc& d, int cfg, hipStream_t stream) {
   constexpr int R = CPLX ? 1 : 2;  // fragments per 32 embedded rows

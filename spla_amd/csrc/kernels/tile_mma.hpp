@@ -63,7 +63,6 @@ namespace tile {
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
-typedef float flt2 __attribute__((ext_vector_type(2)));
 
 template <typename S, int N>
 struct VecOf {

@@ -19,8 +19,6 @@ constexpr double kLaunchSeconds = 4.0e-6;
 
 int blocks_per_cu(int cfg) {
   switch (cfg) {
-    case TileXL:
-      return 1;
     case TileM:
       return 4;
     default:

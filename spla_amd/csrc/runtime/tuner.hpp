@@ -3,10 +3,11 @@
 // A plan is picked by a cost model of the launch: for every tile shape and
 // split factor the model counts the workgroups of the active tiles over the CUs,
 // their time at the shape's sustained MFMA rate, tile padding waste, and the
-// HBM time of the split-K reduction; the cheapest plan wins. Plans are cached
-// per problem key and depend only on the shape, so that repeated calls of one
-// product split the reduction alike and return bitwise identical results (the
-// batch API's plans, by contrast, can be timed: see batched.hpp).
+// HBM time of the split-K reduction; the cheapest plan wins whose sums are no longer
+// than the coarse plan's. Plans are cached per problem key and depend only on the
+// shape, and so do the kernels' sums, however the operands are aligned: repeated
+// calls of one product return bitwise identical results (the batch API's plans, by
+// contrast, can be timed: see batched.hpp).
 // Environment overrides (for tuning sweeps): SPLA_AMD_TILE=L|M|XL,
 // SPLA_AMD_SPLITS=<n>.
 #pragma once
