@@ -5,8 +5,8 @@
 // What bounds it: the matrix cores, and the vector ALU next to them. On gfx950
 // a VALU instruction does not run beside an FP64 or FP32 MFMA of its SIMD: in
 // register-only loops (two waves per SIMD) one v_xor_b32 per MFMA takes
-// v_mfma_f64_16x16x4_f64 from 75.5 to 70.1 TFLOP/s, two to 67.3, four to 64.0
-// (v_mfma_f32_16x16x4_f32: 149, 128, 122, 112), while scalar instructions and
+// v_mfma_f64_16x16x4_f64 from 77.7 to 71.0 TFLOP/s, two to 68.9, four to 65.4
+// (v_mfma_f32_16x16x4_f32: 155, 134, 120, 105), while scalar instructions and
 // one ds_read_b128 per MFMA cost nothing. The k loop is therefore written
 // without vector arithmetic:
 //   * complex operands are not expanded. A fragment holds 16 complex rows (or
@@ -31,7 +31,7 @@
 // Measured against the same tiles with the embedding's swaps and signs, 64-bit
 // addresses and row checks in the loop (one card): complex doubles 2048 x 2048 x
 // 2e5 A^H B 102.3 -> 92.2 ms (72.8 TFLOP/s), 100000 x 4096 x 4096 A B 201.8 ->
-// 176.4 ms (76.1 of the 77.1 a register-only loop reaches), complex floats 2048 x
+// 176.4 ms (76.1 of the 77.7 a register-only loop reaches), complex floats 2048 x
 // 2048 x 2e5 58.9 -> 45.3 ms (148 of 155), real doubles 1000 x 1000 x 1e5 A^T B
 // (ragged) 5.53 -> 3.59 ms.
 //
