@@ -6,7 +6,7 @@
 //   upper: c + nc + colOff > r + rowOff,   lower: r + nr + rowOff > c + colOff.
 // So the active tiles of a tile column are those in front of, or behind, a row that moves
 // by cols from one column to the next: a sum of floors of an arithmetic sequence, which
-// has a closed form as rows and cols divide one another.
+// has a closed form as rows and cols are powers of two.
 //
 // Why not walk the columns: every workgroup looks its tile up, and with hundreds of tile
 // columns the walk outlasts a short product. Measured, walk / closed form: real
@@ -24,18 +24,20 @@ struct FillTiles {
   int mode;        // TileFill, not FillFull
   int64_t off;     // colOff - rowOff
   int64_t m, n;    // elements
-  int rows, cols;  // of a tile; one divides the other
+  int rows, cols;  // of a tile, powers of two
   int64_t tilesM, tilesN;
 
   static constexpr int64_t low(int64_t a, int64_t b) { return a < b ? a : b; }
   static constexpr int64_t high(int64_t a, int64_t b) { return a > b ? a : b; }
-  // quotient of d > 0, rounded up; 0 for a <= 0
-  static constexpr int64_t up(int64_t a, int64_t d) { return a > 0 ? (a + d - 1) / d : 0; }
+  // a / d and the same rounded up (0 for a <= 0) by a power of two; a shift also where the
+  // kernel does not know d beforehand
+  static constexpr int64_t div(int64_t a, int64_t d) { return a >> __builtin_ctzll(d); }
+  static constexpr int64_t up(int64_t a, int64_t d) { return a > 0 ? div(a + d - 1, d) : 0; }
 
   // active tile rows [first_row, end_row) of tile column tn
   constexpr int64_t first_row(int64_t tn) const {
     const int64_t c = tn * cols + off;
-    return mode != FillLower || c <= 0 ? 0 : (c >= m ? tilesM : c / rows);
+    return mode != FillLower || c <= 0 ? 0 : (c >= m ? tilesM : div(c, rows));
   }
   constexpr int64_t end_row(int64_t tn) const {
     return mode != FillUpper ? tilesM : low(tilesM, up(low((tn + 1) * cols, n) + off, rows));
@@ -44,13 +46,13 @@ struct FillTiles {
 
   // sum of floor((u cols + b) / rows) over u < x, b >= 0
   constexpr int64_t floors(int64_t x, int64_t b) const {
-    if (cols >= rows) return x * (x - 1) / 2 * (cols / rows) + x * (b / rows);
-    const int64_t r = rows / cols;
-    return quotients(b / cols + x, r) - quotients(b / cols, r);
+    if (cols >= rows) return x * (x - 1) / 2 * div(cols, rows) + x * div(b, rows);
+    const int64_t r = div(rows, cols);
+    return quotients(div(b, cols) + x, r) - quotients(div(b, cols), r);
   }
   // sum of floor(v / r) over v < y
   static constexpr int64_t quotients(int64_t y, int64_t r) {
-    const int64_t a = y / r;
+    const int64_t a = div(y, r);
     return a * (a - 1) / 2 * r + a * (y - a * r);
   }
 
